@@ -240,44 +240,67 @@ __global__ void k_ls_extrap_list(int stage, const int* list, const int* count, c
   }
 }
 
-// 1/x for x in the normal range: the hardware reciprocal refined by two
-// Newton steps (each doubles the correct bits), within an ulp of the
-// correctly rounded quotient.
+// 1/x for x in the normal range: the hardware reciprocal r (e = 1 - x r of
+// about 2^-27) refined by r (1 + e + e^2), within an ulp of the correctly
+// rounded quotient.
 __device__ __forceinline__ double recip_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// Phi_x_WENO (src/LevelSet/lsTools.cu:9-50).  The level-set kernels let
-// the compiler fuse multiplies and adds (the library is built without
-// contraction elsewhere): they are issue-bound, and the fused forms change
-// results in the last bits only.
-__device__ __forceinline__ double weno5(double b1, double b2, double b3,
-                                        double b4, double b5) {
-#pragma clang fp contract(fast)
-  const double s1 = (13.0 / 12.0) * (b1 - 2.0 * b2 + b3) * (b1 - 2.0 * b2 + b3) +
-                    (0.25) * (b1 - 4.0 * b2 + 3.0 * b3) * (b1 - 4.0 * b2 + 3.0 * b3);
-  const double s2 = (13.0 / 12.0) * (b2 - 2.0 * b3 + b4) * (b2 - 2.0 * b3 + b4) +
-                    (0.25) * (b2 - b4) * (b2 - b4);
-  const double s3 = (13.0 / 12.0) * (b3 - 2.0 * b4 + b5) * (b3 - 2.0 * b4 + b5) +
-                    (0.25) * (3.0 * b3 - 4.0 * b4 + b5) * (3.0 * b3 - 4.0 * b4 + b5);
-  // weights a_k = c_k/d_k, d_k = (s_k + 1e-6)^2, normalised: o_k = c_k p_k /
-  // sum_j c_j p_j with p_k the product of the other two d (one division
-  // instead of four; d_k lies in [1e-12, ~1e16], so the products stay far
-  // from the double range's ends)
-  const double d1 = (s1 + 1.0e-6) * (s1 + 1.0e-6);
-  const double d2 = (s2 + 1.0e-6) * (s2 + 1.0e-6);
-  const double d3 = (s3 + 1.0e-6) * (s3 + 1.0e-6);
-  const double w1 = 0.1 * (d2 * d3), w2 = 0.6 * (d1 * d3), w3 = 0.3 * (d1 * d2);
-  const double isum = recip_nr(w1 + w2 + w3);
-  const double o1 = w1 * isum;
-  const double o2 = w2 * isum;
-  const double o3 = w3 * isum;
-  return ((o1 * (2.0 * b1 - 7.0 * b2 + 11.0 * b3) +
-           o2 * (-1.0 * b2 + 5.0 * b3 + 2.0 * b4) +
-           o3 * (2.0 * b3 + 5.0 * b4 - b5)) *
-          (1.0 / 6.0));
+// 1/sqrt(x) for x in the normal range, by the same third-order step:
+// r (1 + e/2 + 3 e^2/8), e = 1 - x r^2.
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * r, r, 1.0);
+  return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+}
+
+// sqrt(x) for x = 0 or in the normal range: x/sqrt(x) and one residual step.
+__device__ __forceinline__ double sqrt_nr(double x) {
+  const double r = rsqrt_nr(x);
+  const double s = x * r;
+  const double t = __builtin_fma(__builtin_fma(-s, s, x), 0.5 * r, s);
+  return x > 0.0 ? t : x;
+}
+
+// Phi_x_WENO (src/LevelSet/lsTools.cu:9-50), written in the differences
+// e_i = b_{i+1} - b_i of its operands:
+//   4 beta_k = (13/3) dd_k^2 + g_k^2,  dd_k = e_{k+1} - e_k,
+//     g = 3 e2 - e1,  e2 + e3,  3 e3 - e4
+//   6 p_k = 6 b3 + q_k,  q = 5 e2 - 2 e1,  e2 + 2 e3,  4 e3 - e4
+// (p_k the three third-order candidates), so that with weights a_k =
+// c_k/t_k^2 (t_k = 4 (beta_k + 1e-6)) the derivative is
+// b3 + sum(a_k q_k)/(6 sum(a_k)), and with the weights multiplied by
+// (t_1 t_2 t_3)^2 it takes one reciprocal.  42 FP64 instructions (70 as the
+// reference writes the sums).  t_k lies in [4e-6, ~1e9], so the products
+// stay far from the double range's ends.
+__device__ __forceinline__ double weno5_e(double b3, double e1, double e2, double e3, double e4) {
+  const double d1 = e2 - e1, d2 = e3 - e2, d3 = e4 - e3;
+  const double g1 = __builtin_fma(3.0, e2, -e1), g2 = e2 + e3, g3 = __builtin_fma(3.0, e3, -e4);
+  const double t1 = __builtin_fma((13.0 / 3.0) * d1, d1, __builtin_fma(g1, g1, 4.0e-6));
+  const double t2 = __builtin_fma((13.0 / 3.0) * d2, d2, __builtin_fma(g2, g2, 4.0e-6));
+  const double t3 = __builtin_fma((13.0 / 3.0) * d3, d3, __builtin_fma(g3, g3, 4.0e-6));
+  const double u1 = t2 * t3, u2 = t1 * t3, u3 = t1 * t2;
+  const double w1 = u1 * u1, w2 = 6.0 * (u2 * u2), w3 = 3.0 * (u3 * u3);
+  const double q1 = __builtin_fma(2.0, g1, -e2), q2 = g2 + e3, q3 = g3 + e3;
+  const double num = __builtin_fma(w1, q1, __builtin_fma(w2, q2, w3 * q3));
+  return __builtin_fma(num * (1.0 / 6.0), recip_nr(w1 + w2 + w3), b3);
+}
+
+// Whether any of the three candidates 6 b3 + q_k may be positive (a NaN
+// counts as one).
+__device__ __forceinline__ bool weno5_positive(double b3, double e1, double e2, double e3,
+                                               double e4) {
+  const double lim = -6.0 * b3;
+  const double q1 = __builtin_fma(5.0, e2, -2.0 * e1), q2 = __builtin_fma(2.0, e3, e2),
+               q3 = __builtin_fma(4.0, e3, -e4);
+  return !(q1 <= lim && q2 <= lim && q3 <= lim);
+}
+
+__device__ __forceinline__ double weno5(double b1, double b2, double b3, double b4, double b5) {
+  return weno5_e(b3, b2 - b1, b3 - b2, b4 - b3, b5 - b4);
 }
 
 // Backward difference of phi along axis `ax` at point (x,y,z), with the
@@ -481,82 +504,201 @@ __device__ __forceinline__ int mirror_images(int X, int n, int c[3]) {
   return k;
 }
 
-// One SSP-RK3 stage of the reinitialisation at every padded point: the two
-// JB WENO derivatives per axis, the Godunov |grad phi| by the sign of phi0
-// and rs = S(phi0)(|grad phi| - 1), S = phi0/sqrt(phi0^2 + dmin^2)
-// (reini_RS_WENOJB, lsTools.cu:824-900), then RunGK_{First,Second,Third}S
+// One axis of the Godunov gradient, max(max(L, 0), max(-R, 0)), from the
+// axis' six metric-scaled differences bd (offsets -2..+3) multiplied by
+// sign(phi0).  (With that sign s, the reference's max(max(L,0)^2, min(R,0)^2)
+// for s > 0 and max(max(R,0)^2, min(L,0)^2) for s < 0 are both the square
+// of this.)  L takes bd[0..4] (the fifth given as l5), R takes bd[5..1].
+// A WENO derivative is a convex combination of its three candidates, so a
+// side whose candidates are all <= 0 (left) or all >= 0 (right) gives 0
+// and is not formed.  Away from kinks of phi that is one of the two
+// sides: the operands of the side that counts are selected and one
+// derivative is evaluated; a second one only where a lane of the wavefront
+// needs both.  The differences e of R's operands are L's in the opposite
+// order and sign, so -R = -bd[3] + (the sum L adds to its b3).
+__device__ __forceinline__ double godunov_axis(const double bd[6], double l5) {
+  const double e1 = bd[1] - bd[0], e2 = bd[2] - bd[1], e3 = bd[3] - bd[2], e4 = l5 - bd[3],
+               r4 = bd[4] - bd[3], r5 = bd[5] - bd[4];
+  const bool left = weno5_positive(bd[2], e1, e2, e3, e4);
+  const bool right = weno5_positive(-bd[3], r5, r4, e3, e2);
+  const double v = weno5_e(left ? bd[2] : -bd[3], left ? e1 : r5, left ? e2 : r4, e3,
+                           left ? e4 : e2);
+  double c = v > 0.0 ? v : 0.0;
+  if (left && right) {
+    const double r = weno5_e(-bd[3], r5, r4, e3, e2);
+    c = r > c ? r : c;
+  }
+  return c;
+}
+
+// The edge rules of axis_bd, stencil_left and stencil_right at position q of
+// n, applied to the six differences: past the low face the first one is
+// repeated, past the high face they are mirrored.
+__device__ __forceinline__ void edge_bd(double bd[6], int q, int n) {
+  if (q == 0) bd[2] = bd[3];
+  if (q <= 1) bd[1] = bd[2];
+  if (q <= 2) bd[0] = bd[1];
+  if (q == n - 1) bd[3] = bd[2];
+  if (q == n - 1) bd[4] = bd[1];
+  if (q == n - 2) bd[4] = bd[3];
+  if (q == n - 1) bd[5] = bd[0];
+  if (q == n - 2) bd[5] = bd[2];
+  if (q == n - 3) bd[5] = bd[4];
+}
+
+// One SSP-RK3 stage of the reinitialisation: the two JB WENO derivatives per
+// axis, the Godunov |grad phi| by the sign of phi0 and rs = S(phi0)
+// (|grad phi| - 1), S = phi0/sqrt(phi0^2 + dmin^2) (reini_RS_WENOJB,
+// lsTools.cu:824-900), then RunGK_{First,Second,Third}S
 // (extrapol.cu:155-212).  src is the stage input, P the iteration's phi,
 // which is also its phi0 (the reference copies phi to phi0 at the start of
-// every iteration).  The last stage computes the interior points and writes
-// each into out, a different array, together with its mirror images in the
-// ghost layers: out is then the next iteration's phi with the ghost
-// mirroring that iteration would start with already applied.
-__global__ void k_ls_reinit_stage(int stage, const double* src, const double* P,
-                                  const double* dmin, const double* j1, const double* j5,
-                                  const double* j9, PDims g, double iX, double iY, double iZ,
-                                  double dt, double* out) {
-  const long long NG = g.N();
-  const double* P0 = P;
-  for (long long id = (long long)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-       id < NG; id += (long long)gridDim.x * blockDim.x) {
-    const unsigned uid = (unsigned)id, row = uid / (unsigned)g.x;  // NG < 2^32
-    const int x = (int)(uid - row * (unsigned)g.x), y = (int)(row % (unsigned)g.y),
-              z = (int)(row / (unsigned)g.y);
-    if (stage == 2 && (x < GC || x >= g.x - GC || y < GC || y >= g.y - GC || z < GC ||
-                       z >= g.z - GC))
-      continue;  // a ghost point: written as an interior point's image
-    const double ih[3] = {iX, iY, iZ};
-    const double met[3] = {j1[id], j5[id], j9[id]};
-    const double p0 = P0[id];
-    const double ta = (double)(p0 > 0.0) - (double)(p0 < 0.0);
-    double r[3];
+// every iteration).  Stage 0 computes every padded point, stage 1 all but
+// the two outermost ghost layers (the last stage's stencils do not reach
+// them), stage 2 the interior points, each written into out, a different
+// array, together with its mirror images in the ghost layers: out is then
+// the next iteration's phi with the ghost mirroring that iteration would
+// start with already applied.
+//
+// A workgroup owns a 32 x 8 tile of (x, y) and marches z through a slab of
+// kz planes with the stencil's z values and differences in registers, so a
+// point loads 13 values of src instead of 21 and the index arithmetic is
+// done once per column.  Bound by instruction issue (about 400 VALU
+// instructions per point-wave, the issue slots 80% busy) with the memory
+// floor (56 B per padded point) close behind: 97 us a stage at 218 x 186 x
+// 170 padded points, 4.1 TB/s, against 182 us for the form with one point
+// per work-item and both WENO derivatives of every axis.  Wider tiles waste
+// lanes at the row ends (64 x 4: 10% slower), 16 x 16 tiles 3%; loading the
+// next plane's streamed fields ahead costs the registers of a fifth
+// wavefront and was 4% slower.  The four fields no stage writes take
+// nontemporal loads, which leaves the last-level cache to phi (1% faster).
+constexpr int RI_TX = 32, RI_TY = 8;
+
+template <int STAGE>
+__global__ void __launch_bounds__(256)
+k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const double* j1,
+                  const double* j5, const double* j9, PDims g, int kz, double iX, double iY,
+                  double iZ, double dt, double* out) {
+  constexpr int LO = STAGE == 0 ? 0 : (STAGE == 1 ? GC - 3 : GC);
+  const int nbx = (g.x - 2 * LO + RI_TX - 1) / RI_TX, nby = (g.y - 2 * LO + RI_TY - 1) / RI_TY;
+  const int b = (int)xcd_block(blockIdx.x, gridDim.x);
+  const int x = LO + (b % nbx) * RI_TX + (int)threadIdx.x % RI_TX;
+  const int y = LO + (b / nbx % nby) * RI_TY + (int)threadIdx.x / RI_TX;
+  const int z0 = LO + b / (nbx * nby) * kz, z1 = min(z0 + kz, g.z - LO);
+  const bool own = x < g.x - LO && y < g.y - LO;
+  // work-items past the tile's end follow the last column and store nothing
+  const int xc = min(x, g.x - 1 - LO), yc = min(y, g.y - 1 - LO);
+  const unsigned sy = (unsigned)g.x, sz = (unsigned)g.x * (unsigned)g.y;  // NG < 2^32
+  const unsigned col = (unsigned)xc + sy * (unsigned)yc;
+  // stencil positions past the padded grid's faces, clamped (their
+  // differences are never used); none in stage 2
+  const bool edge_x = STAGE < 2 && __any(xc < 3 || xc > g.x - 4);
+  const bool edge_y = STAGE < 2 && __any(yc < 3 || yc > g.y - 4);
+  auto clampz = [&](int z) { return STAGE < 2 ? min(max(z, 0), g.z - 1) : z; };
+  // a field's value at byte offset off (the padded grid has fewer than 2^29
+  // points): uniform base, 32-bit offset
+  auto at = [](const double* f, unsigned off) {
+    return reinterpret_cast<const double*>(reinterpret_cast<const char*>(f) + off);
+  };
+  auto ld = [&](const double* f, unsigned off) { return *at(f, off); };
+  auto ldn = [&](const double* f, unsigned off) { return __builtin_nontemporal_load(at(f, off)); };
+  auto plane = [&](int z) { return ld(src, (col + (unsigned)clampz(z) * sz) * 8u); };
+  double vz[4], dz[6];  // values of planes z .. z+3; the stencil's differences along z
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const int pos[3] = {x, y, z}, ext[3] = {g.x, g.y, g.z};
-      const unsigned stride[3] = {1u, (unsigned)g.x, (unsigned)g.x * (unsigned)g.y};
-      double bd[6], L, R;
-      if (pos[c] >= 3 && pos[c] <= ext[c] - 4) {
-        // away from the padded grid's faces: the interior operands, left
-        // (q-2..q+2) and right (q+3..q-1) biased, with no edge rules
-        axis_bd_inner(src, stride[c], uid, ih[c], met[c], bd);
-        L = weno5(bd[0], bd[1], bd[2], bd[3], bd[4]);
-        R = weno5(bd[5], bd[4], bd[3], bd[2], bd[1]);
-      } else {
-        double b[5];
-        axis_bd(src, stride[c], pos[c], ext[c], uid, ih[c], met[c], bd);
-        stencil_left(src, g, c, pos[c], ext[c], x, y, z, ih[c], met[c], bd, b);
-        L = weno5(b[0], b[1], b[2], b[3], b[4]);
-        stencil_right(pos[c], ext[c], bd, b);
-        R = weno5(b[0], b[1], b[2], b[3], b[4]);
-      }
-      const double lp = L > 0.0 ? L : 0.0, rm = R < 0.0 ? R : 0.0;
-      double hi = lp * lp, lo = rm * rm;
-      r[c] = 0.5 * (ta + 1.0) * (hi > lo ? hi : lo);
-      const double rp = R > 0.0 ? R : 0.0, lm = L < 0.0 ? L : 0.0;
-      hi = rp * rp;
-      lo = lm * lm;
-      r[c] += 0.5 * fabs(ta - 1.0) * (hi > lo ? hi : lo);
+  for (int o = 0; o < 3; o++) vz[o + 1] = plane(z0 + o);
+  {
+    const double a = plane(z0 - 3), b2 = plane(z0 - 2), c = plane(z0 - 1);
+    dz[1] = b2 - a;
+    dz[2] = c - b2;
+    dz[3] = vz[1] - c;
+    dz[4] = vz[2] - vz[1];
+    dz[5] = vz[3] - vz[2];
+  }
+  for (int z = z0; z < z1; z++) {
+#pragma unroll
+    for (int o = 0; o < 3; o++) vz[o] = vz[o + 1];
+#pragma unroll
+    for (int o = 0; o < 5; o++) dz[o] = dz[o + 1];
+    vz[3] = plane(z + 3);
+    dz[5] = vz[3] - vz[2];
+    const unsigned id = col + (unsigned)z * sz, off = id * 8u;
+    const double sv = vz[0];
+    double vx[7], vy[7];
+#pragma unroll
+    for (int o = 0; o < 7; o++) {
+      if (o == 3) vx[o] = vy[o] = sv;
+      else if (edge_x) vx[o] = ld(src, (id + (unsigned)(min(max(xc - 3 + o, 0), g.x - 1) - xc)) * 8u);
+      else vx[o] = ld(src + (o - 3), off);
     }
-    const double grad_mod = sqrt(r[0] + r[1] + r[2]);
-    const double d = dmin[id];
-    const double so = p0 / sqrt(p0 * p0 + d * d);
-    const double rs = 1.0 * so * (grad_mod - 1.0);
-    const double sv = src[id];
-    if (stage == 0) {
-      out[id] = sv - dt * rs;
-    } else if (stage == 1) {
-      out[id] = 0.75 * P[id] + 0.25 * (sv - dt * rs);
+#pragma unroll
+    for (int o = 0; o < 7; o++) {
+      if (o == 3) continue;
+      if (edge_y) vy[o] = ld(src, (id + (unsigned)(min(max(yc - 3 + o, 0), g.y - 1) - yc) * sy) * 8u);
+      else vy[o] = ld(src + (o - 3) * (int)sy, off);
+    }
+    const double p0 = STAGE == 0 ? sv : ld(P, off);
+    // metric / spacing with the sign of phi0 (at phi0 = 0, S and with it rs
+    // vanish)
+    auto signed_by_p0 = [&](double s) {
+      return __longlong_as_double(__double_as_longlong(s) ^
+                                  (__double_as_longlong(p0) & (long long)(1ull << 63)));
+    };
+    const double sx = signed_by_p0(iX * ldn(j1, off)), sY = signed_by_p0(iY * ldn(j5, off)),
+                 sZ = signed_by_p0(iZ * ldn(j9, off)), d = ldn(dmin, off);
+    double bx[6], by[6], bz[6];
+#pragma unroll
+    for (int o = 0; o < 6; o++) {
+      bx[o] = sx * (vx[o + 1] - vx[o]);
+      by[o] = sY * (vy[o + 1] - vy[o]);
+      bz[o] = sZ * dz[o];
+    }
+    if (edge_x) edge_bd(bx, xc, g.x);
+    if (edge_y) edge_bd(by, yc, g.y);
+    double z5 = bz[4];
+    if (STAGE < 2 && (z < 3 || z > g.z - 4)) {
+      edge_bd(bz, z, g.z);
+      // on the last plane L's fifth operand is the z difference one row down
+      // (id_kp2 = id_jm1, lsTools.cu:636)
+      z5 = z == g.z - 1 ? bdiff(src, g, 2, xc, yc == 0 ? yc : yc - 1, z, sZ) : bz[4];
+    }
+    const double rx = godunov_axis(bx, bx[4]), ry = godunov_axis(by, by[4]),
+                 rz = godunov_axis(bz, z5);
+    const double grad = sqrt_nr(__builtin_fma(rx, rx, __builtin_fma(ry, ry, rz * rz)));
+    const double so = p0 * rsqrt_nr(__builtin_fma(p0, p0, d * d));
+    const double step = __builtin_fma(-dt * so, grad - 1.0, sv);  // sv - dt*rs
+    if (!own) continue;
+    if constexpr (STAGE == 0) {
+      out[id] = step;
+    } else if constexpr (STAGE == 1) {
+      out[id] = 0.75 * p0 + 0.25 * step;
     } else {
-      const double o = (P[id] + 2.0 * (sv - dt * rs)) / 3.0;
+      // (P + 2 step)/3, the quotient corrected by its residual
+      const double t = p0 + 2.0 * step, o3 = t * (1.0 / 3.0);
+      const double o = __builtin_fma(__builtin_fma(-3.0, o3, t), 1.0 / 3.0, o3);
       int cx[3], cy[3], cz[3];
       const int kx = mirror_images(x, g.x - 2 * GC, cx), ky = mirror_images(y, g.y - 2 * GC, cy),
-                kz = mirror_images(z, g.z - 2 * GC, cz);
-      for (int c = 0; c < kz; c++)
-        for (int b = 0; b < ky; b++)
+                kk = mirror_images(z, g.z - 2 * GC, cz);
+      for (int c = 0; c < kk; c++)
+        for (int e = 0; e < ky; e++)
           for (int a = 0; a < kx; a++)
-            out[(unsigned)cx[a] + (unsigned)g.x * ((unsigned)cy[b] + (unsigned)g.y * (unsigned)cz[c])] = o;
+            out[(unsigned)cx[a] + sy * (unsigned)cy[e] + sz * (unsigned)cz[c]] = o;
     }
   }
+}
+
+template <int STAGE>
+void launch_reinit_stage(hipStream_t st, const double* src, const double* P, const double* dmin,
+                         const double* j1, const double* j5, const double* j9, PDims g, double iX,
+                         double iY, double iZ, double dt, double* out) {
+  constexpr int LO = STAGE == 0 ? 0 : (STAGE == 1 ? GC - 3 : GC);
+  const long long cols = (long long)((g.x - 2 * LO + RI_TX - 1) / RI_TX) *
+                         ((g.y - 2 * LO + RI_TY - 1) / RI_TY);
+  const int nz = g.z - 2 * LO;
+  // 8 planes a slab (16: 4% slower, a longer last round of workgroups), fewer
+  // while the chip's 256 compute units would get less than four workgroups
+  int kz = 8;
+  while (kz > 2 && cols * ((nz + kz - 1) / kz) < 1024) kz /= 2;
+  hipLaunchKernelGGL(k_ls_reinit_stage<STAGE>, dim3((unsigned)(cols * ((nz + kz - 1) / kz))),
+                     dim3(256), 0, st, src, P, dmin, j1, j5, j9, g, kz, iX, iY, iZ, dt, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -738,14 +880,11 @@ int op_ls_reinit(emx_ctx* ctx, double* phi, const double* jbn, const double* dmi
   for (int it = 1; it <= 10; it++) {
     // per point: src, three metrics, phi (= phi0), dmin, out
     EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              hipLaunchKernelGGL(k_ls_reinit_stage, dim3(bg), dim3(256), 0, st, 0, P, P, Dm,
-                                 J1, J5, J9, g, iX, iY, iZ, dt, T1));
+              launch_reinit_stage<0>(st, P, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, T1));
     EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              hipLaunchKernelGGL(k_ls_reinit_stage, dim3(bg), dim3(256), 0, st, 1, T1, P, Dm,
-                                 J1, J5, J9, g, iX, iY, iZ, dt, T2));
+              launch_reinit_stage<1>(st, T1, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, T2));
     EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              hipLaunchKernelGGL(k_ls_reinit_stage, dim3(bg), dim3(256), 0, st, 2, T2, P, Dm,
-                                 J1, J5, J9, g, iX, iY, iZ, dt, Q));
+              launch_reinit_stage<2>(st, T2, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, Q));
     double* t = P;
     P = Q;
     Q = t;
