@@ -21,6 +21,8 @@
 // derivatives per point (store), so flux formation, metric projection and
 // the accumulation of the divergence are fused into the solve.
 #pragma once
+#include <type_traits>
+
 #include "emx_internal.hpp"
 
 namespace emx {
@@ -129,6 +131,42 @@ struct chunk_store<Prob, decltype(void(Prob::CHUNK_STORE))> {
   static constexpr bool value = Prob::CHUNK_STORE;
 };
 
+// LINE_STORE: the problem stores a lane's C points of a line of the wavefront
+// kind at once (store_line<C>), reading what its stores need first.
+template <class Prob, class = void>
+struct line_store { static constexpr bool value = false; };
+template <class Prob>
+struct line_store<Prob, decltype(void(Prob::LINE_STORE))> {
+  static constexpr bool value = Prob::LINE_STORE;
+};
+
+// INTERLEAVE: the parts (below) read fields in common, so the parts of a
+// line group run next to each other.
+template <class Prob, class = void>
+struct interleaves { static constexpr bool value = false; };
+template <class Prob>
+struct interleaves<Prob, decltype(void(Prob::INTERLEAVE))> {
+  static constexpr bool value = Prob::INTERLEAVE;
+};
+
+// Part: the problem stands for several independent ones of type Part, one
+// per z block of a launch (part(z), z < parts(); NV and BATCH_STORE are the
+// part's).
+template <class Prob, class = void>
+struct parts_of {
+  static constexpr bool many = false;
+  static int count(const Prob&) { return 1; }
+  static __device__ __forceinline__ const Prob& get(const Prob& p, int) { return p; }
+};
+template <class Prob>
+struct parts_of<Prob, std::void_t<typename Prob::Part>> {
+  static constexpr bool many = true;
+  static int count(const Prob& p) { return p.parts(); }
+  static __device__ __forceinline__ typename Prob::Part get(const Prob& p, int z) {
+    return p.part(z);
+  }
+};
+
 __device__ __forceinline__ int clampi(int v, int lo, int hi) {
   return v < lo ? lo : (v > hi ? hi : v);
 }
@@ -194,87 +232,122 @@ __device__ __forceinline__ void stage_wave_tabs(const LineTab& T, double* lds) {
 
 // Solves NV fields of one line held by a wavefront in the coalesced order
 // (v[q][a]: point q*64 + lane of field a), in place: each field moves to
-// the chunk order through the wave's LDS buffer xb, takes the local
-// forward and backward sweeps and the carry scans, and moves back.
-template <int S, int C, int NV>
+// the chunk order through the wave's LDS buffer xb (F*64*(C+1) doubles),
+// takes the local forward and backward sweeps and the carry scans, and moves
+// back.  F fields at a time share one chain of LDS and lane-exchange waits.
+template <int S, int C, int NV, int F>
 __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& wt, double* xb,
                                            int n, int P, double ih, int lane) {
+  static_assert(NV % F == 0, "fields per group");
   constexpr int H = scheme_halo<S>::value;
   constexpr int W = C + 2 * H;
+  constexpr int XS = 64 * (C + 1);
   const int s = lane * C;
   const bool act = lane < P;
 #pragma unroll
-  for (int a = 0; a < NV; a++) {
+  for (int a = 0; a < NV; a += F) {
     // to the chunk order
     wave_sync();
 #pragma unroll
     for (int q = 0; q < C; q++) {
       const int idx = q * 64 + lane;
-      xb[idx + idx / C] = v[q][a];
+#pragma unroll
+      for (int f = 0; f < F; f++) xb[f * XS + idx + idx / C] = v[q][a + f];
     }
     wave_sync();
-    double w[W];
+    double w[F][W];
 #pragma unroll
     for (int q = 0; q < W; q++) {
       const int l = clampi(s - H + q, 0, n - 1);
-      w[q] = xb[l + l / C];
+#pragma unroll
+      for (int f = 0; f < F; f++) w[f][q] = xb[f * XS + l + l / C];
     }
     // local forward sweep from a zero carry
-    double y[C];
-    double yp = 0.0;
+    double y[F][C], yp[F];
+#pragma unroll
+    for (int f = 0; f < F; f++) yp[f] = 0.0;
 #pragma unroll
     for (int q = 0; q < C; q++) {
       const int l = s + q;
       if (act && l < n) {
-        const double r = line_rhs<S>(&w[q + H], l, n, ih);
-        yp = r * wt.ib[q * 64 + lane] - wt.m[q * 64 + lane] * yp;
-        y[q] = yp;
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+          const double r = line_rhs<S>(&w[f][q + H], l, n, ih);
+          yp[f] = r * wt.ib[q * 64 + lane] - wt.m[q * 64 + lane] * yp[f];
+          y[f][q] = yp[f];
+        }
       } else {
-        y[q] = 0.0;
+#pragma unroll
+        for (int f = 0; f < F; f++) y[f][q] = 0.0;
       }
     }
     // forward carries: inclusive weighted scan over lanes
     {
-      double B = act ? yp : 0.0;
+      double B[F];
+#pragma unroll
+      for (int f = 0; f < F; f++) B[f] = act ? yp[f] : 0.0;
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
-        const double up = __shfl_up(B, d, 64);
-        if (lane >= d) B += wt.af[k * 64 + lane] * up;
-      }
-      double Y = __shfl_up(B, 1, 64);
-      if (lane == 0) Y = 0.0;
+        double up[F];
 #pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (act && l < n) y[q] += wt.H[q * 64 + lane] * Y;
+        for (int f = 0; f < F; f++) up[f] = __shfl_up(B[f], d, 64);
+        if (lane >= d) {
+#pragma unroll
+          for (int f = 0; f < F; f++) B[f] += wt.af[k * 64 + lane] * up[f];
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        double Y = __shfl_up(B[f], 1, 64);
+        if (lane == 0) Y = 0.0;
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+          const int l = s + q;
+          if (act && l < n) y[f][q] += wt.H[q * 64 + lane] * Y;
+        }
       }
     }
     // local backward sweep from a zero carry
-    double xs = 0.0;
+    double xs[F];
+#pragma unroll
+    for (int f = 0; f < F; f++) xs[f] = 0.0;
 #pragma unroll
     for (int q = C - 1; q >= 0; q--) {
       const int l = s + q;
       if (act && l < n) {
-        xs = y[q] - wt.gam1[q * 64 + lane] * xs;
-        y[q] = xs;
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+          xs[f] = y[f][q] - wt.gam1[q * 64 + lane] * xs[f];
+          y[f][q] = xs[f];
+        }
       }
     }
     // backward carries: weighted scan from the right, then the result
     {
-      double B = act ? xs : 0.0;
+      double B[F];
+#pragma unroll
+      for (int f = 0; f < F; f++) B[f] = act ? xs[f] : 0.0;
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
-        const double dn = __shfl_down(B, d, 64);
-        if (lane + d < 64) B += wt.ab[k * 64 + lane] * dn;
-      }
-      double X = __shfl_down(B, 1, 64);
-      if (lane == 63) X = 0.0;
+        double dn[F];
 #pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (act && l < n) y[q] += wt.G[q * 64 + lane] * X;
+        for (int f = 0; f < F; f++) dn[f] = __shfl_down(B[f], d, 64);
+        if (lane + d < 64) {
+#pragma unroll
+          for (int f = 0; f < F; f++) B[f] += wt.ab[k * 64 + lane] * dn[f];
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        double X = __shfl_down(B[f], 1, 64);
+        if (lane == 63) X = 0.0;
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+          const int l = s + q;
+          if (act && l < n) y[f][q] += wt.G[q * 64 + lane] * X;
+        }
       }
     }
     // back to the coalesced order
@@ -282,16 +355,26 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
 #pragma unroll
     for (int q = 0; q < C; q++) {
       const int l = s + q;
-      if (act && l < n) xb[l + l / C] = y[q];
+      if (act && l < n) {
+#pragma unroll
+        for (int f = 0; f < F; f++) xb[f * XS + l + l / C] = y[f][q];
+      }
     }
     wave_sync();
 #pragma unroll
     for (int q = 0; q < C; q++) {
       const int idx = q * 64 + lane;
-      v[q][a] = xb[idx + idx / C];
+#pragma unroll
+      for (int f = 0; f < F; f++) v[q][a + f] = xb[f * XS + idx + idx / C];
     }
   }
 }
+
+// Fields the wavefront kind solves side by side on one grid: with one point
+// per lane the waits of a solve outweigh its arithmetic, and the registers
+// are there.
+template <int C, int NV>
+constexpr int wave_group() { return C == 1 && NV <= 4 ? NV : (C == 2 && NV % 2 == 0 ? 2 : 1); }
 
 // ---------------------------------------------------------------------------
 // One wavefront per line (xi lines, contiguous in memory).  Lines are
@@ -305,14 +388,14 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
 // q*64 + lane, so the 64 lanes read 64 consecutive doubles (no bank
 // conflicts), and the backward factor is stored shifted (entry l holds
 // gamma[l+1]).
-template <int S, int C, class Prob>
+template <int S, int C, class Prob, int F = 1>
 __device__ __forceinline__ void lines_wave_body(const Prob& prob, const LineTab& T,
                                                 long long nlines, int nyl, long long sj,
                                                 long long sk, long long sl, double ih,
                                                 long long blk, long long nblk) {
   constexpr int NV = Prob::NV;
   constexpr bool PRE = prefetches<Prob>::value;
-  constexpr int STR = C + 1;  // chunk stride in the transpose buffer
+  constexpr int STR = F * (C + 1);  // transpose buffer, doubles per lane
   constexpr int TS = 64 * C;  // per-point table stride (chunk order)
   extern __shared__ double lds[];
   const int n = T.n, P = T.P;
@@ -354,12 +437,16 @@ __device__ __forceinline__ void lines_wave_body(const Prob& prob, const LineTab&
     if constexpr (PRE) {
       if (more) load_line(Ln, vn);
     }
-    wave_solve<S, C, NV>(v, wt, xb, n, P, ih, lane);
+    wave_solve<S, C, NV, F>(v, wt, xb, n, P, ih, lane);
     const long long bs = line_base(L);
+    if constexpr (line_store<Prob>::value) {
+      prob.template store_line<C>(bs, sl, lane, n, v);
+    } else {
 #pragma unroll
-    for (int q = 0; q < C; q++) {
-      const int idx = q * 64 + lane;
-      if (idx < n) prob.store(bs + (long long)idx * sl, v[q]);
+      for (int q = 0; q < C; q++) {
+        const int idx = q * 64 + lane;
+        if (idx < n) prob.store(bs + (long long)idx * sl, v[q]);
+      }
     }
     if (!more) break;
     L = Ln;
@@ -378,7 +465,8 @@ template <int S, int C, class Prob>
 __global__ void __launch_bounds__(256)
 k_lines_wave(Prob prob, LineTab T, long long nlines, int nyl, long long sj,
              long long sk, long long sl, double ih) {
-  lines_wave_body<S, C>(prob, T, nlines, nyl, sj, sk, sl, ih, blockIdx.x, gridDim.x);
+  lines_wave_body<S, C, Prob, wave_group<C, Prob::NV>()>(prob, T, nlines, nyl, sj, sk, sl, ih,
+                                                        blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -467,16 +555,23 @@ __device__ __forceinline__ void lines_strided_body(const Prob& prob, const LineT
   }
   __syncthreads();
   if (act) {
+    // the fields' sums side by side: one chain of LDS waits, not NV
     const int kk = c < K ? c : K;
+    double Y[NV];
 #pragma unroll
-    for (int a = 0; a < NV; a++) {
-      double Y = 0.0;
-      for (int k = 0; k < kk; k++)
-        Y += s_wf[c * KB + k] * sh[(a * P + c - 1 - k) * LG + li];
+    for (int a = 0; a < NV; a++) Y[a] = 0.0;
+    for (int k = 0; k < kk; k++) {
+      const double wf = s_wf[c * KB + k];
 #pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (l < n) y[a][q] += s_H[l] * Y;
+      for (int a = 0; a < NV; a++) Y[a] += wf * sh[(a * P + c - 1 - k) * LG + li];
+    }
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+      const int l = s + q;
+      if (l < n) {
+        const double Hl = s_H[l];
+#pragma unroll
+        for (int a = 0; a < NV; a++) y[a][q] += Hl * Y[a];
       }
     }
   }
@@ -506,11 +601,11 @@ __device__ __forceinline__ void lines_strided_body(const Prob& prob, const LineT
   const int kb = P - 1 - c < K ? P - 1 - c : K;
   double X[NV];
 #pragma unroll
-  for (int a = 0; a < NV; a++) {
-    double acc = 0.0;
-    for (int k = 0; k < kb; k++)
-      acc += s_wb[c * KB + k] * sh[(a * P + c + 1 + k) * LG + li];
-    X[a] = acc;
+  for (int a = 0; a < NV; a++) X[a] = 0.0;
+  for (int k = 0; k < kb; k++) {
+    const double wb = s_wb[c * KB + k];
+#pragma unroll
+    for (int a = 0; a < NV; a++) X[a] += wb * sh[(a * P + c + 1 + k) * LG + li];
   }
   if constexpr (batch_store<Prob>::value && C % 4 == 0) {
     // groups of four points, each stored by one store_batch where the whole
@@ -555,28 +650,6 @@ __device__ __forceinline__ void lines_strided_body(const Prob& prob, const LineT
   }
 }
 
-template <int S, int C, int LG, class Prob>
-__global__ void __launch_bounds__(1024)
-k_lines_strided(Prob prob, LineTab T, int nlanes, long long si, long long so,
-                long long sl, double ih) {
-  lines_strided_body<S, C, LG>(prob, T, nlanes, si, so, sl, ih,
-                               line_group<LG>(blockIdx.x, gridDim.x), blockIdx.y);
-}
-
-// ---------------------------------------------------------------------------
-// Many grids in one launch: workgroup b belongs to the grid g with
-// blk_start[g] <= b < blk_start[g+1] and solves that grid's line group
-// (b - blk_start[g]) % gx, outer index (b - blk_start[g]) / gx.  Each grid
-// has its own table (line length), geometry and problem data.
-template <class Prob>
-struct BatchLines {
-  Prob prob;
-  LineTab T;
-  int nlanes, gx;
-  long long si, so, sl;
-  double ih;
-};
-
 // Workgroup local (of ngroup in its grid) -> line group g, row-major over
 // (group along the lines, outer index).  A grid's rows start anywhere in a
 // 128-byte cache line (its nx is any size), so neighbouring groups along a
@@ -595,6 +668,48 @@ __device__ __forceinline__ int xcd_run_group(int local, int ngroup) {
   if (r >= 8 * k) return local;
   return base + (r & 7) * k + (r >> 3);
 }
+
+// run: line groups are dealt by xcd_run_group, for launches of more
+// workgroups than the chip holds at once.  Rows that start inside a cache
+// line share it with their neighbours (stage at 187 x 151 x 129: 1183 us
+// round robin, 1139 us in runs), and where they do not, a run's neighbouring
+// segments still arrive in order (256^3: 4165 and 4073 us).  A small launch
+// would only pay for the divisions (64^3 gradient and divergence: 43.2 us
+// round robin, 43.7 us in runs).
+template <int S, int C, int LG, class Prob>
+__global__ void __launch_bounds__(1024)
+k_lines_strided(Prob prob, LineTab T, int nlanes, long long si, long long so,
+                long long sl, double ih, int run) {
+  int part = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
+  if (run) {
+    int g;
+    if constexpr (interleaves<Prob>::value) {
+      g = xcd_run_group(bx + gridDim.x * (by + gridDim.y * part),
+                        gridDim.x * gridDim.y * gridDim.z);
+      part = g % gridDim.z;
+      g /= gridDim.z;
+    } else {
+      g = xcd_run_group(bx + gridDim.x * by, gridDim.x * gridDim.y);
+    }
+    bx = g % gridDim.x;
+    by = g / gridDim.x;
+  }
+  lines_strided_body<S, C, LG>(parts_of<Prob>::get(prob, part), T, nlanes, si, so, sl, ih, bx, by);
+}
+
+// ---------------------------------------------------------------------------
+// Many grids in one launch: workgroup b belongs to the grid g with
+// blk_start[g] <= b < blk_start[g+1] and solves that grid's line group
+// (b - blk_start[g]) % gx, outer index (b - blk_start[g]) / gx.  Each grid
+// has its own table (line length), geometry and problem data.
+template <class Prob>
+struct BatchLines {
+  Prob prob;
+  LineTab T;
+  int nlanes, gx;
+  long long si, so, sl;
+  double ih;
+};
 
 // MAXT: the largest workgroup the launch uses.  1024 serves lines of up to
 // 512 points at any shape; 256 (lines of up to 256/LG chunks) lets a
@@ -971,7 +1086,8 @@ template <int S, int C, class Prob>
 hipError_t launch_wave_c(const Prob& prob, const LineTab& T, const DirGeom& g,
                          double ih, hipStream_t st) {
   // one resident set of workgroups; each wave takes every (4*blocks)-th line
-  const size_t lds = (size_t)(5 * 64 * C + 768 + 4 * 64 * (C + 1)) * sizeof(double);
+  const size_t lds = (size_t)(5 * 64 * C + 768 + 4 * 64 * wave_group<C, Prob::NV>() * (C + 1)) *
+                     sizeof(double);
   if (lds > 65536)
     (void)hipFuncSetAttribute((const void*)k_lines_wave<S, C, Prob>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -982,6 +1098,19 @@ hipError_t launch_wave_c(const Prob& prob, const LineTab& T, const DirGeom& g,
                      dim3(256), lds, st, prob, T, g.nlines, g.nyl, g.sj, g.sk,
                      g.sl, ih);
   return hipGetLastError();
+}
+
+template <int S, class Prob>
+hipError_t launch_wave_s(const Prob& prob, const LineTab& T, const DirGeom& g, double ih,
+                         hipStream_t st) {
+  switch (T.C) {
+    case 1: return launch_wave_c<S, 1>(prob, T, g, ih, st);
+    case 2: return launch_wave_c<S, 2>(prob, T, g, ih, st);
+    case 4: return launch_wave_c<S, 4>(prob, T, g, ih, st);
+    case 8: return launch_wave_c<S, 8>(prob, T, g, ih, st);
+    case 16: return launch_wave_c<S, 16>(prob, T, g, ih, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int S, int C, int LG, class Prob>
@@ -1001,11 +1130,13 @@ hipError_t launch_strided_c(const Prob& prob, const LineTab& T,
   } else {
   const size_t lds = (size_t)(5 * T.n + 1 + 2 * T.P * T.KB +
                               Prob::NV * T.P * LG) * sizeof(double);
+  grid.z = parts_of<Prob>::count(prob);
+  const int run = (long long)grid.x * grid.y * grid.z > 1024;
   if (lds > 65536)
     (void)hipFuncSetAttribute((const void*)k_lines_strided<S, C, LG, Prob>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((k_lines_strided<S, C, LG, Prob>), grid, dim3(threads), lds,
-                     st, prob, T, g.nlanes, g.si, g.so, g.sl, ih);
+  hipLaunchKernelGGL((k_lines_strided<S, C, LG, Prob>), grid, dim3(threads), lds, st, prob, T,
+                     g.nlanes, g.si, g.so, g.sl, ih, run);
   return hipGetLastError();
   }
 }
@@ -1019,14 +1150,7 @@ hipError_t launch_lines_s(const Prob& prob, const LineTab& T, const DirGeom& g,
     // work-item's chunk must fit its registers)
     switch (T.kind) {
       case KIND_WAVE:
-        switch (T.C) {
-          case 1: return launch_wave_c<S, 1>(prob, T, g, ih, st);
-          case 2: return launch_wave_c<S, 2>(prob, T, g, ih, st);
-          case 4: return launch_wave_c<S, 4>(prob, T, g, ih, st);
-          case 8: return launch_wave_c<S, 8>(prob, T, g, ih, st);
-          case 16: return launch_wave_c<S, 16>(prob, T, g, ih, st);
-        }
-        break;
+        return launch_wave_s<S>(prob, T, g, ih, st);
       case KIND_STRIDED32:
         if (T.C == 4) return launch_strided_c<S, 4, 32>(prob, T, g, ih, st);
         if (T.C == 8) return launch_strided_c<S, 8, 32>(prob, T, g, ih, st);
@@ -1041,27 +1165,23 @@ hipError_t launch_lines_s(const Prob& prob, const LineTab& T, const DirGeom& g,
         break;
     }
     return hipErrorInvalidValue;
-  } else if constexpr (Prob::NV > 4) {
-    // more than four solves per work-item only fit the wavefront kind
+  } else if constexpr (Prob::NV >= 4) {
+    // four solves per work-item only fit the wavefront kind (on the strided
+    // kinds they spill up to 484 bytes a work-item at chunks of 16)
     if (T.kind != KIND_WAVE) return hipErrorInvalidValue;
-    switch (T.C) {
-      case 1: return launch_wave_c<S, 1>(prob, T, g, ih, st);
-      case 2: return launch_wave_c<S, 2>(prob, T, g, ih, st);
-      case 4: return launch_wave_c<S, 4>(prob, T, g, ih, st);
-      case 8: return launch_wave_c<S, 8>(prob, T, g, ih, st);
-    }
-    return hipErrorInvalidValue;
+    return launch_wave_s<S>(prob, T, g, ih, st);
   } else {
     switch (T.kind) {
       case KIND_WAVE:
-        switch (T.C) {
-          case 1: return launch_wave_c<S, 1>(prob, T, g, ih, st);
-          case 2: return launch_wave_c<S, 2>(prob, T, g, ih, st);
-          case 4: return launch_wave_c<S, 4>(prob, T, g, ih, st);
-          case 8: return launch_wave_c<S, 8>(prob, T, g, ih, st);
-          case 16: return launch_wave_c<S, 16>(prob, T, g, ih, st);
+        if constexpr (parts_of<Prob>::many) {
+          // this kind's workgroups are persistent: one launch per part
+          hipError_t e = hipSuccess;
+          for (int z = 0; e == hipSuccess && z < prob.parts(); z++)
+            e = launch_wave_s<S>(prob.part(z), T, g, ih, st);
+          return e;
+        } else {
+          return launch_wave_s<S>(prob, T, g, ih, st);
         }
-        break;
       case KIND_STRIDED:
         switch (T.C) {
           case 8: return launch_strided_c<S, 8, 64>(prob, T, g, ih, st);

@@ -96,6 +96,69 @@ struct ProbGradDiv {
   }
 };
 
+// ProbGradDiv in two halves, (u, v) and (w, the projected velocity), which
+// the strided kinds solve as parts of one launch: the same values and
+// arithmetic, two solves per work-item.
+struct ProbGradDivHalf {
+  static constexpr int NV = 2;
+  static constexpr bool BATCH_STORE = true;
+  ProbGradDiv g;
+  int half;
+  __device__ __forceinline__ void load(long long p, double* v) const {
+    const long long N = g.N;
+    if (half == 0) {
+      v[0] = g.u[p];
+      v[1] = g.u[N + p];
+    } else {
+      v[0] = g.u[2 * N + p];
+      v[1] = g.jbn[9 * N + p] * (g.jbn[4 * g.dir * N + p] * g.u[g.dir * N + p]);
+    }
+  }
+  __device__ __forceinline__ void store(long long p, const double* v) const {
+    store_batch<1>(p, 0, reinterpret_cast<const double(*)[NV]>(v));
+  }
+  template <int Q>
+  __device__ __forceinline__ void store_batch(long long p, long long sl,
+                                              const double (*v)[NV]) const {
+    const long long N = g.N;
+    double* d = g.dvel + (3 * g.dir + 2 * half) * N + p;
+    if (half == 0) {
+#pragma unroll
+      for (int i = 0; i < Q; i++) {
+        d[i * sl] = v[i][0];
+        d[N + i * sl] = v[i][1];
+      }
+      return;
+    }
+    double a[Q], q[Q];
+    if (g.dir > 0) {
+#pragma unroll
+      for (int i = 0; i < Q; i++) {
+        a[i] = g.acc[p + i * sl];
+        q[i] = g.dir == 2 ? g.jbn[10 * N + p + i * sl] : 0.0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < Q; i++) {
+      d[i * sl] = v[i][0];
+      if (g.dir == 0) g.acc[p + i * sl] = v[i][1];
+      else if (g.dir == 1) g.acc[p + i * sl] = a[i] + v[i][1];
+      else g.div[p + i * sl] = q[i] * (a[i] + v[i][1]);
+    }
+  }
+};
+
+struct ProbGradDivParts {
+  using Part = ProbGradDivHalf;
+  static constexpr int NV = 2;
+  static constexpr bool BATCH_STORE = true, INTERLEAVE = true;  // both halves read u_dir
+  static const char* label() { return ProbGradDiv::label(); }
+  double bytes_pt() const { return g.bytes_pt(); }
+  ProbGradDiv g;
+  static int parts() { return 2; }
+  __host__ __device__ __forceinline__ Part part(int z) const { return Part{g, z}; }
+};
+
 // Inputs of flujos (solver/flujos_compact.f90) addressed by linear index.
 struct FluxIn {
   const double* um;    // 5 comps
@@ -382,6 +445,42 @@ struct ProbAccum {
       __builtin_nontemporal_store(q * (acc[N + p] + v[1]), &out1[p]);
     }
   }
+};
+
+// The eight projected fluxes of one direction as four ProbAccum pairs,
+// outputs rs 1..5 then rsv 2..4, in one launch of the strided kinds: four
+// launches of a coarse grid do not fill the chip (64 x 56 x 48: 8.8 us each,
+// 11.4 us together).
+struct ProbAccumAll {
+  using Part = ProbAccum;
+  static constexpr int NV = ProbAccum::NV;
+  static constexpr bool BATCH_STORE = true;
+  static const char* label() { return ProbAccum::label(); }
+  double bytes_pt() const { return 4.0 * part(0).bytes_pt(); }
+  const double* f;  // 8 slots (stride N)
+  double* acc;
+  double* rs;
+  double* rsv;
+  const double* ij;
+  long long N;
+  int pass;
+  static int parts() { return 4; }
+  __host__ __device__ __forceinline__ Part part(int z) const {
+    const int slot = 2 * z;
+    return Part{f + slot * N, acc + slot * N, slot < 5 ? rs + slot * N : rsv + (slot - 4) * N,
+                slot + 1 < 5 ? rs + (slot + 1) * N : rsv + (slot - 3) * N, ij, N, pass};
+  }
+};
+
+// The derivatives of four fields as two pairs, likewise.
+struct ProbDerivPairs {
+  using Part = ProbDeriv<2>;
+  static constexpr int NV = 2;
+  static const char* label() { return Part::label(); }
+  double bytes_pt() const { return 64.0; }
+  ProbDeriv<2> lo, hi;
+  static int parts() { return 2; }
+  __host__ __device__ __forceinline__ Part part(int z) const { return z == 0 ? lo : hi; }
 };
 
 inline unsigned pointwise_blocks(long long n) {

@@ -68,6 +68,16 @@ static int deriv_fields(emx_ctx* ctx, int dir, int m, const double* const* in,
     }
     return launch_lines(ctx, dir, p, ih);
   }
+  if (m == 4) {
+    ProbDerivPairs p;
+    for (int a = 0; a < 2; a++) {
+      p.lo.in[a] = in[a];
+      p.lo.out[a] = out[a];
+      p.hi.in[a] = in[2 + a];
+      p.hi.out[a] = out[2 + a];
+    }
+    return launch_lines(ctx, dir, p, ih);
+  }
   for (; f + 1 < m; f += 2) {
     ProbDeriv<2> p;
     p.in[0] = in[f];
@@ -119,7 +129,8 @@ int op_grad_div(emx_ctx* ctx, const double* u, const double* jbn, double* dvel, 
   const long long N = ctx->d.N();
   for (int d = 0; d < 3; d++) {
     ProbGradDiv p{u, jbn, dvel, ctx->acc, div, N, d};
-    EMX_TRY(launch_lines(ctx, d, p, ih[d]));
+    if (ctx->plan[PLAN_DERIV][d].kind == KIND_WAVE) EMX_TRY(launch_lines(ctx, d, p, ih[d]));
+    else EMX_TRY(launch_lines(ctx, d, ProbGradDivParts{p}, ih[d]));
   }
   return EMX_OK;
 }

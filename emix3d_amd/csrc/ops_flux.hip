@@ -9,6 +9,14 @@ __global__ void k_fill(double* a, double v, long long n) {
     a[p] = v;
 }
 
+// Two fields set to v (blockIdx.y selects).
+__global__ void k_fill2(double* a, double* b, double v, long long n) {
+  double* f = blockIdx.y == 0 ? a : b;
+  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < n;
+       p += (long long)gridDim.x * blockDim.x)
+    f[p] = v;
+}
+
 __global__ void k_flujos(FluxIn F, int neq, double* flux) {
   const long long N = F.N;
   for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < N;
@@ -147,7 +155,7 @@ k_flux_project_xi(FluxIn F, LineTab T, long long nlines, int nx, int ny, int yz,
 #pragma unroll
       for (int a = 0; a < 2; a++) v[q][a] = lineF[(2 * wv + a) * TS + idc];
     }
-    wave_solve<S, C, 2>(v, wt, xb, n, P, ih, lane);
+    wave_solve<S, C, 2, 1>(v, wt, xb, n, P, ih, lane);
 #pragma unroll
     for (int q = 0; q < C; q++) {
       const int idx = q * 64 + lane;
@@ -306,17 +314,11 @@ int op_flux_div_all(emx_ctx* ctx, const FluxPtrs& fp, const double ih[3],
   int pass = fused_xi ? 1 : 0, k = fused_xi ? 1 : 0;
   for (int dir = fused_xi ? 1 : 0; dir < 3; dir++) {
     if (!(mat & (1 << dir))) continue;
-    // slots (0,1) (2,3) (4,5) (6,7): outputs rs 1..5 then rsv 2..4.  (Four
-    // slots per launch, which reads 1/J once per four fluxes in the last
-    // pass, measured 1.6x slower per flux on the 32-lines-per-wave kind:
-    // twice the values per work-item.)
-    for (int slot = 0; slot < 8; slot += 2) {
-      double* o0 = slot < 5 ? rs + slot * N : rsv + (slot - 4) * N;
-      double* o1 = slot + 1 < 5 ? rs + (slot + 1) * N : rsv + (slot - 3) * N;
-      ProbAccum p{ctx->fluxbuf + (8 * k + slot) * N, ctx->acc + slot * N, o0, o1,
-                  fp.jbn + 10 * N, N, pass};
-      EMX_TRY(launch_lines(ctx, dir, p, ih[dir]));
-    }
+    // slots in pairs.  (Four slots per work-item, which reads 1/J once per
+    // four fluxes in the last pass, measured 1.6x slower per flux on the
+    // 32-lines-per-wave kind: twice the values per work-item.)
+    const ProbAccumAll p{ctx->fluxbuf + 8 * k * N, ctx->acc, rs, rsv, fp.jbn + 10 * N, N, pass};
+    EMX_TRY(launch_lines(ctx, dir, p, ih[dir]));
     k++;
     pass++;
   }
@@ -337,12 +339,9 @@ int op_flux_div_all(emx_ctx* ctx, const FluxPtrs& fp, const double ih[3],
     pass++;
   }
   // zero viscous divergence of the continuity and scalar equations
-  EMX_TIMED(ctx, "fill", 8.0 * N,
-          hipLaunchKernelGGL(k_fill, dim3(pointwise_blocks(N)), dim3(256), 0,
-                     ctx->stream, rsv, 0.0, N));
-  EMX_TIMED(ctx, "fill", 8.0 * N,
-          hipLaunchKernelGGL(k_fill, dim3(pointwise_blocks(N)), dim3(256), 0,
-                     ctx->stream, rsv + 4 * N, 0.0, N));
+  EMX_TIMED(ctx, "fill", 16.0 * N,
+          hipLaunchKernelGGL(k_fill2, dim3(pointwise_blocks(N), 2), dim3(256), 0,
+                     ctx->stream, rsv, rsv + 4 * N, 0.0, N));
   EMX_TRY_HIP(hipGetLastError());
   return EMX_OK;
 }
