@@ -38,6 +38,52 @@ struct ProbFilter {
   }
 };
 
+// The five conservative fields (stride N) in one launch.  The strided kinds
+// take them as parts, a line group's five next to each other on one XCD: J
+// and 1/J come from memory once and from its L2 four times (96 B per point
+// and direction instead of 160).
+struct ProbFilterParts {
+  using Part = ProbFilter;
+  static constexpr int NV = 1;
+  static constexpr bool BATCH_STORE = true, INTERLEAVE = true;
+  double* f;
+  const double* jac;
+  const double* ijac;
+  long long N;
+  static int parts() { return 5; }
+  __host__ __device__ __forceinline__ Part part(int m) const { return Part{f + m * N, jac, ijac}; }
+};
+
+// The wavefront kind solves a line's five fields one after another, J and
+// 1/J read once for all.  Same arithmetic as ProbFilter.
+struct ProbFilterLine {
+  static constexpr int NV = 5;
+  static constexpr bool PREFETCH = true, LINE_STORE = true;
+  double* f;
+  const double* jac;
+  const double* ijac;
+  long long N;
+  __device__ __forceinline__ void load(long long p, double* v) const {
+    const double j = jac[p];
+#pragma unroll
+    for (int m = 0; m < 5; m++) v[m] = f[m * N + p] * j;
+  }
+  template <int C>
+  __device__ __forceinline__ void store_line(long long base, long long sl, int lane, int n,
+                                             const double (*v)[NV]) const {
+    double q[C];
+#pragma unroll
+    for (int i = 0; i < C; i++) q[i] = ijac[base + min(i * 64 + lane, n - 1) * sl];
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+      if (i * 64 + lane >= n) continue;
+#pragma unroll
+      for (int m = 0; m < 5; m++)
+        __builtin_nontemporal_store(v[i][m] * q[i], &f[m * N + base + (i * 64 + lane) * sl]);
+    }
+  }
+};
+
 namespace {
 
 // xi: one wavefront per line, the shortest chunk that covers the line;
@@ -47,7 +93,7 @@ int filter_shape(int dir, int n, int* kind, int* C) {
     int c = 1;
     while (c * 64 < n) c *= 2;
     *kind = KIND_WAVE;
-    *C = c;
+    *C = c == 4 && n <= 192 ? 3 : c;
   } else {
     *kind = KIND_STRIDED32;
     *C = 16;
@@ -56,18 +102,28 @@ int filter_shape(int dir, int n, int* kind, int* C) {
 }
 
 template <int S>
-hipError_t launch_filter(const ProbFilter& p, const LineTab& T, const DirGeom& g, double cfilt,
-                         hipStream_t st) {
+hipError_t launch_filter(double* um1, const double* jbn, long long N, const LineTab& T,
+                         const DirGeom& g, double cfilt, hipStream_t st) {
+  const double *jac = jbn + 9 * N, *ijac = jbn + 10 * N;
   if (T.kind == KIND_WAVE) {
+    const ProbFilterLine p{um1, jac, ijac, N};
     switch (T.C) {
       case 1: return launch_wave_c<S, 1>(p, T, g, cfilt, st);
       case 2: return launch_wave_c<S, 2>(p, T, g, cfilt, st);
+      case 3: return launch_wave_c<S, 3>(p, T, g, cfilt, st);
       case 4: return launch_wave_c<S, 4>(p, T, g, cfilt, st);
-      case 8: return launch_wave_c<S, 8>(p, T, g, cfilt, st);
-      default: return launch_wave_c<S, 16>(p, T, g, cfilt, st);
     }
+    // lines past 256 points: five fields of such a chunk do not fit the
+    // registers
+    hipError_t e = hipSuccess;
+    for (int m = 0; e == hipSuccess && m < 5; m++) {
+      const ProbFilter q{um1 + m * N, jac, ijac};
+      e = T.C == 8 ? launch_wave_c<S, 8>(q, T, g, cfilt, st)
+                   : launch_wave_c<S, 16>(q, T, g, cfilt, st);
+    }
+    return e;
   }
-  return launch_strided_c<S, 16, 32>(p, T, g, cfilt, st);
+  return launch_strided_c<S, 16, 32>(ProbFilterParts{um1, jac, ijac, N}, T, g, cfilt, st);
 }
 
 }  // namespace
@@ -88,15 +144,14 @@ int op_filtrado(emx_ctx* ctx, int itf, double* um1, const double* jbn, double cf
   for (int k = 0; k < 3; k++) {
     const int dir = order[itf - 1][k];
     const DirGeom g = dir_geom(ctx->d, dir);
-    for (int m = 0; m < 5; m++) {
-      ProbFilter p{um1 + m * N, jbn + 9 * N, jbn + 10 * N};
-      LaunchTimer timer(ctx, ProbFilter::label(), dir, p.bytes_pt() * (double)N);
-      const hipError_t e = dir == 2 ? launch_filter<FILTER_P>(p, tab[dir], g, cfilt, ctx->stream)
-                                    : launch_filter<FILTER_NP>(p, tab[dir], g, cfilt, ctx->stream);
-      if (e != hipSuccess) {
-        set_error("filter launch (dir %d) failed: %s", dir, hipGetErrorString(e));
-        return EMX_ERR_HIP;
-      }
+    // five fields in and out, J and 1/J
+    LaunchTimer timer(ctx, ProbFilter::label(), dir, 96.0 * (double)N);
+    const hipError_t e =
+        dir == 2 ? launch_filter<FILTER_P>(um1, jbn, N, tab[dir], g, cfilt, ctx->stream)
+                 : launch_filter<FILTER_NP>(um1, jbn, N, tab[dir], g, cfilt, ctx->stream);
+    if (e != hipSuccess) {
+      set_error("filter launch (dir %d) failed: %s", dir, hipGetErrorString(e));
+      return EMX_ERR_HIP;
     }
   }
   // u, temp, pres from the filtered variables (herramientas_incomp2.f90:395-405)
