@@ -122,15 +122,6 @@ struct batch_store<Prob, decltype(void(Prob::BATCH_STORE))> {
   static constexpr bool value = Prob::BATCH_STORE;
 };
 
-// CHUNK_STORE: the problem scatters a work-item's whole chunk at once
-// (store_w<C>), used where the chunk is contiguous in memory.
-template <class Prob, class = void>
-struct chunk_store { static constexpr bool value = false; };
-template <class Prob>
-struct chunk_store<Prob, decltype(void(Prob::CHUNK_STORE))> {
-  static constexpr bool value = Prob::CHUNK_STORE;
-};
-
 // LINE_STORE: the problem stores a lane's C points of a line of the wavefront
 // kind at once (store_line<C>), reading what its stores need first.
 template <class Prob, class = void>
@@ -165,6 +156,17 @@ struct parts_of<Prob, std::void_t<typename Prob::Part>> {
   static __device__ __forceinline__ typename Prob::Part get(const Prob& p, int z) {
     return p.part(z);
   }
+};
+
+// ADJ_WAVES: wavefronts per SIMD the problem's transposed solve of four-point
+// chunks is compiled for.  Six (80 registers) hold three workgroups of
+// 128-point lines on a CU (the flux adjoint's solve at 128^3: 110 us with
+// four, 100 us with six); a scatter that would spill there takes four.
+template <class Prob, class = void>
+struct adj_waves { static constexpr int value = 6; };
+template <class Prob>
+struct adj_waves<Prob, decltype(void(Prob::ADJ_WAVES))> {
+  static constexpr int value = Prob::ADJ_WAVES;
 };
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) {
@@ -892,148 +894,222 @@ k_lines_tile(Prob prob, LineTab T, int nlanes, long long si, long long so,
 // ---------------------------------------------------------------------------
 // Transposed compact derivative along lines: out = (ih A^{-1} B)^T g
 // = ih B^T A^{-T} g.  T is a TAB_TRANSPOSED table: the Thomas factors and
-// chunk-carry weights of A^T, and B^T as seven diagonals.  Each work-item
-// solves its chunk of A^T y = g (carries as in k_lines_tile), the solution
-// goes to an LDS tile [n][LG] of the field, and B^T is applied from the
-// tile.  The NV fields of a point are solved one after another.  Launch
-// geometry of k_lines_tile.
-// CHUNK (xi lines, contiguous in memory; problems with CHUNK_STORE): the
-// scatter of a work-item's chunk goes through store_w<C> (k_lines_adj_xi).
-template <int C, int LG, class Prob, bool CHUNK>
+// chunk-carry weights of A^T, and B^T as seven diagonals.  A work-item
+// solves its chunk of A^T y = g for all NV fields side by side, in the
+// registers of the values it loaded; the solutions then go field by field
+// through an LDS tile [n][LG] (two in turn, one barrier per field) for the
+// B^T stencil.  Problem interface: load(p, v) one point, load_w<C>(p, v) C
+// adjacent points, store<C>(p, stride, m, v) the first m of C points.
+//
+// Bound by LDS reads when every field was solved by itself: 116 reads of 8
+// bytes per field and four-point chunk (the Thomas factors and all 28
+// stencil coefficients and rows again for each field).  Side by side the
+// factors and carry weights are read once for all fields, the interior rows
+// of B^T, which are equal, are in scalar registers, and the chunk's own rows
+// are not read back: about 50 reads.  The gradient's adjoint
+// at 128^3: 56 us a direction before, 42-46 us now (3.3 TB/s).
+constexpr int ADJ_EDGE = 4;  // rows at either end of B^T that differ
+
+template <int C, int LG, bool XI, class Prob>
 __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& T, int nlanes,
                                                long long si, long long so, long long sl,
-                                               double ih) {
+                                               double ih, int bx, int by) {
   constexpr int NV = Prob::NV;
-  constexpr int PMAX = 1024 / LG;
   extern __shared__ double lds[];
   const int n = T.n, P = T.P, K = T.K, KB = T.KB;
   const int ntab = 5 * n + 1;
+  const int region = max(NV * P, n) * LG;
   double* s_ib = lds;
   double* s_m = s_ib + n;
   double* s_gam = s_m + n;
   double* s_H = s_gam + n + 1;
   double* s_G = s_H + n;
-  double* s_wf = s_G + n;         // [P*KB]
-  double* s_wb = s_wf + P * KB;   // [P*KB]
-  double* s_bt = s_wb + P * KB;   // [7n]
-  double* sh = s_bt + 7 * n;      // [PMAX][LG] carries
-  double* tile = sh + PMAX * LG;  // [n][LG]
+  double* s_wf = s_G + n;               // [P*KB]
+  double* s_wb = s_wf + P * KB;         // [P*KB]
+  double* s_be = s_wb + P * KB;         // [2*ADJ_EDGE][7]: rows 0..3 and n-4..n-1 of B^T
+  double* rA = s_be + 2 * ADJ_EDGE * 7; // forward carries [NV][P][LG], then tile [n][LG]
+  double* rB = rA + region;             // backward carries, then tile
   const int tid = threadIdx.x;
   const int li = tid % LG;
   const int c = tid / LG;
-  const int i = blockIdx.x * LG + li;
+  const int i = line_group<LG>(bx, gridDim.x) * LG + li;
   const bool act = i < nlanes && c < P;
   const int ic = i < nlanes ? i : nlanes - 1;
-  const long long base = (long long)ic * si + (long long)blockIdx.y * so;
+  const long long base = (long long)ic * si + (long long)by * so;
   const int s = c * C;
+  const int m = min(C, n - s);  // points of this chunk (<= 0: none)
 
   double v[C][NV];
+  bool loaded = false;
+  if constexpr (XI) {
+    if (m == C) {
+      prob.template load_w<C>(base + s, v);
+      loaded = true;
+    }
+  }
+  if (!loaded) {
 #pragma unroll
-  for (int q = 0; q < C; q++) {
-    const int l = s + q < n ? s + q : n - 1;
-    prob.load(base + (long long)l * sl, v[q]);
+    for (int q = 0; q < C; q++) {
+      const int l = s + q < n ? s + q : n - 1;
+      prob.load(base + (long long)l * sl, v[q]);
+    }
   }
   {
     const int nstage = ntab + 2 * P * KB;
     const int woff = (int)(T.WfB - T.blob);
     for (int t = tid; t < nstage; t += blockDim.x)
       lds[t] = gref(T.blob + (t < ntab ? t : t - ntab + woff));
-    for (int t = tid; t < 7 * n; t += blockDim.x) s_bt[t] = T.BT[t];
+    for (int t = tid; t < 2 * ADJ_EDGE * 7; t += blockDim.x) {
+      const int e = t / 7, row = e < ADJ_EDGE ? e : n - 2 * ADJ_EDGE + e;
+      s_be[t] = gref(T.BT + 7 * row + t % 7);
+    }
   }
+  // the interior row of B^T (its outermost diagonals are zero)
+  double bt[5];
 #pragma unroll
-  for (int a = 0; a < NV; a++) {
-    __syncthreads();
-    double y[C];
-    double yp = 0.0;
+  for (int k = 0; k < 5; k++) bt[k] = gref(T.BT + 7 * (n / 2) + 1 + k);
+  __syncthreads();
+  if (act) {
 #pragma unroll
     for (int q = 0; q < C; q++) {
-      const int l = s + q;
-      if (act && l < n) {
-        yp = v[q][a] * s_ib[l] - s_m[l] * yp;
-        y[q] = yp;
-      } else {
-        y[q] = 0.0;
-      }
-    }
-    sh[c * LG + li] = act ? yp : 0.0;
-    __syncthreads();
-    if (act) {
-      const int kk = c < K ? c : K;
-      double Y = 0.0;
-      for (int k = 0; k < kk; k++) Y += s_wf[c * KB + k] * sh[(c - 1 - k) * LG + li];
+      if (q < m) {
+        const double ib = s_ib[s + q], sm = s_m[s + q];
 #pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (l < n) y[q] += s_H[l] * Y;
+        for (int a = 0; a < NV; a++) v[q][a] = v[q][a] * ib - sm * (q > 0 ? v[q - 1][a] : 0.0);
+      } else {
+#pragma unroll
+        for (int a = 0; a < NV; a++) v[q][a] = q > 0 ? v[q - 1][a] : 0.0;  // the last value
       }
     }
-    double xs = 0.0;
+  }
+  if (c < P) {
+#pragma unroll
+    for (int a = 0; a < NV; a++) rA[(a * P + c) * LG + li] = act ? v[C - 1][a] : 0.0;
+  }
+  __syncthreads();
+  if (act) {
+    double Y[NV];
+#pragma unroll
+    for (int a = 0; a < NV; a++) Y[a] = 0.0;
+    const int kk = c < K ? c : K;
+    for (int k = 0; k < kk; k++) {
+      const double w = s_wf[c * KB + k];
+#pragma unroll
+      for (int a = 0; a < NV; a++) Y[a] += w * rA[(a * P + c - 1 - k) * LG + li];
+    }
 #pragma unroll
     for (int q = C - 1; q >= 0; q--) {
-      const int l = s + q;
-      if (act && l < n) {
-        xs = y[q] - s_gam[l + 1] * xs;
-        y[q] = xs;
-      }
-    }
-    __syncthreads();
-    sh[c * LG + li] = act ? xs : 0.0;
-    __syncthreads();
-    if (act) {
-      const int kb = P - 1 - c < K ? P - 1 - c : K;
-      double X = 0.0;
-      for (int k = 0; k < kb; k++) X += s_wb[c * KB + k] * sh[(c + 1 + k) * LG + li];
+      if (q < m) {
+        const double h = s_H[s + q], gam = s_gam[s + q + 1];
 #pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (l < n) tile[l * LG + li] = y[q] + s_G[l] * X;
-      }
-    }
-    __syncthreads();
-    if (act) {
-#pragma unroll
-      for (int q = 0; q < C; q++) {
-        const int l = s + q;
-        if (l < n) {
-          double r = 0.0;
-#pragma unroll
-          for (int k = 0; k < 7; k++) {
-            const int t = l + k - 3;
-            if (t >= 0 && t < n) r += s_bt[7 * l + k] * tile[t * LG + li];
-          }
-          v[q][a] = ih * r;
+        for (int a = 0; a < NV; a++) {
+          v[q][a] += h * Y[a];
+          if (q < C - 1) v[q][a] -= gam * (q + 1 < m ? v[q + 1][a] : 0.0);
         }
       }
     }
   }
-  if (!act) return;  // after the last barrier
-  if constexpr (CHUNK) {
-    if (s + C <= n) {  // the chunk's C points are adjacent (unit stride)
-      prob.template store_w<C>(base + s, v);
-      return;
+  if (c < P) {
+#pragma unroll
+    for (int a = 0; a < NV; a++) rB[(a * P + c) * LG + li] = act ? v[0][a] : 0.0;
+  }
+  __syncthreads();
+  if (act) {
+    double X[NV];
+#pragma unroll
+    for (int a = 0; a < NV; a++) X[a] = 0.0;
+    const int kb = P - 1 - c < K ? P - 1 - c : K;
+    for (int k = 0; k < kb; k++) {
+      const double w = s_wb[c * KB + k];
+#pragma unroll
+      for (int a = 0; a < NV; a++) X[a] += w * rB[(a * P + c + 1 + k) * LG + li];
+    }
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+      if (q < m) {
+        const double g = s_G[s + q];
+#pragma unroll
+        for (int a = 0; a < NV; a++) v[q][a] += g * X[a];
+      }
     }
   }
+  const bool inner = s >= ADJ_EDGE && s + C <= n - ADJ_EDGE;
 #pragma unroll
-  for (int q = 0; q < C; q++) {
-    const int l = s + q;
-    if (l < n) prob.store(base + (long long)l * sl, v[q]);
+  for (int a = 0; a < NV; a++) {
+    // a tile is written again two fields later, past a barrier that follows
+    // its readers; the forward and backward carries lie a barrier back too
+    double* tile = (a & 1 ? rB : rA) + li;
+    if (act) {
+#pragma unroll
+      for (int q = 0; q < C; q++)
+        if (q < m) tile[(s + q) * LG] = v[q][a];
+    }
+    __syncthreads();
+    if (act) {
+      if (inner) {
+        double w[C + 4];
+        w[0] = tile[(s - 2) * LG];
+        w[1] = tile[(s - 1) * LG];
+        w[C + 2] = tile[(s + C) * LG];
+        w[C + 3] = tile[(s + C + 1) * LG];
+#pragma unroll
+        for (int q = 0; q < C; q++) w[q + 2] = v[q][a];
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+          double r = 0.0;
+#pragma unroll
+          for (int k = 0; k < 5; k++) r += bt[k] * w[q + k];
+          v[q][a] = ih * r;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+          const int l = s + q;
+          if (q < m) {
+            const bool edge = l < ADJ_EDGE || l >= n - ADJ_EDGE;
+            const double* be = s_be + 7 * (l < ADJ_EDGE ? l : l - (n - 2 * ADJ_EDGE));
+            double r = 0.0;
+#pragma unroll
+            for (int k = 0; k < 7; k++) {
+              const int t = l + k - 3;
+              if (t >= 0 && t < n) {
+                const double b = edge ? be[k] : (k > 0 && k < 6 ? bt[k - 1] : 0.0);
+                r += b * tile[t * LG];
+              }
+            }
+            v[q][a] = ih * r;
+          }
+        }
+      }
+    }
   }
+  if (act && m > 0) prob.template store<C, XI>(base + (long long)s * sl, XI ? 1 : sl, m, v);
 }
 
-template <int C, int LG, class Prob>
-__global__ void __launch_bounds__(1024)
+// Parts and run as in k_lines_strided.  Lines of up to 256 points take chunks
+// of four and 16 lines per workgroup (8 lines: 119 us for the solve at 128^3
+// against 100 us, the tables being staged twice as often), up to 512 points
+// chunks of eight and 8 lines, as two tiles of 16 lines of 512 points would
+// take all of a CU's LDS.
+template <int C, int LG, bool XI, class Prob>
+__global__ void __launch_bounds__(C == 4 && LG == 16 ? 1024 : 512) __attribute__((amdgpu_waves_per_eu(C == 4 ? adj_waves<Prob>::value : 2)))
 k_lines_adj(Prob prob, LineTab T, int nlanes, long long si, long long so, long long sl,
-            double ih) {
-  lines_adj_body<C, LG, Prob, false>(prob, T, nlanes, si, so, sl, ih);
-}
-
-// The xi form: at most 256 work-items per workgroup and three waves per
-// SIMD, which leaves the chunk scatter the registers of its C points.
-template <int C, int LG, class Prob>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_lines_adj_xi(Prob prob, LineTab T, int nlanes, long long si, long long so, long long sl,
-               double ih) {
-  lines_adj_body<C, LG, Prob, true>(prob, T, nlanes, si, so, sl, ih);
+            double ih, int run) {
+  int part = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
+  if (run) {
+    int g;
+    if constexpr (interleaves<Prob>::value) {
+      g = xcd_run_group(bx + gridDim.x * (by + gridDim.y * part),
+                        gridDim.x * gridDim.y * gridDim.z);
+      part = g % gridDim.z;
+      g /= gridDim.z;
+    } else {
+      g = xcd_run_group(bx + gridDim.x * by, gridDim.x * gridDim.y);
+    }
+    bx = g % gridDim.x;
+    by = g / gridDim.x;
+  }
+  lines_adj_body<C, LG, XI>(parts_of<Prob>::get(prob, part), T, nlanes, si, so, sl, ih, bx, by);
 }
 
 // ---------------------------------------------------------------------------
@@ -1234,49 +1310,37 @@ int launch_lines(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
   return EMX_OK;
 }
 
-// Longest line of the transposed solve (its LDS tile holds a whole line of
-// 16 lanes).
+// Longest line of the transposed solve (its LDS tiles hold whole lines).
 constexpr int ADJ_MAX_N = 512;
 
-// Chunk length of the transposed solve (16 lines per wavefront).
+// Chunk length of the transposed solve.
 inline int adj_chunk(int n) { return n <= 256 ? 4 : 8; }
 
 // Solve all lines of direction dir with the transposed operator; T is the
 // context's TAB_TRANSPOSED table of that direction.
-template <class Prob>
-int launch_lines_adj(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
+template <bool XI, class Prob>
+int launch_lines_adj_as(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
   const DirGeom g = dir_geom(ctx->d, dir);
   const LineTab& T = ctx->adj[dir];
   LaunchTimer timer(ctx, Prob::label(), dir, prob.bytes_pt() * (double)ctx->d.N());
+  using Part = std::decay_t<decltype(parts_of<Prob>::get(prob, 0))>;
   auto go = [&](auto kern, int LG) {
-    dim3 grid((g.nlanes + LG - 1) / LG, g.nouter);
+    dim3 grid((g.nlanes + LG - 1) / LG, g.nouter, parts_of<Prob>::count(prob));
     const int threads = ((T.P * LG + 63) / 64) * 64;
-    const size_t lds = (size_t)(5 * T.n + 1 + 2 * T.P * T.KB + 7 * T.n + (1024 / LG) * LG +
-                                T.n * LG) * sizeof(double);
+    const size_t lds = (size_t)(5 * T.n + 1 + 2 * T.P * T.KB + 2 * ADJ_EDGE * 7 +
+                                2 * std::max(Part::NV * T.P, T.n) * LG) * sizeof(double);
     if (lds > 65536)
       (void)hipFuncSetAttribute((const void*)kern,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, grid, dim3(threads), lds, ctx->stream, prob, T, g.nlanes,
-                       g.si, g.so, g.sl, ih);
+                       g.si, g.so, g.sl, ih, (int)((long long)grid.x * grid.y * grid.z > 1024));
   };
-  // xi lines of a chunk-scattering problem with chunks of four (lines of up
-  // to 256): as many lines per workgroup (4, 8 or 16) as keep it within
-  // 256 items, so the chunk scatter has the registers of such a workgroup
-  // (with chunks of eight it does not fit them); otherwise 16 lines per
-  // workgroup and the point-by-point scatter
-  bool chunked = false;
-  if constexpr (chunk_store<Prob>::value) {
-    if (g.sl == 1 && T.C == 4 && T.P <= 64) {
-      const int lg = T.P <= 16 ? 16 : (T.P <= 32 ? 8 : 4);
-      if (lg == 16) go(k_lines_adj_xi<4, 16, Prob>, 16);
-      else if (lg == 8) go(k_lines_adj_xi<4, 8, Prob>, 8);
-      else go(k_lines_adj_xi<4, 4, Prob>, 4);
-      chunked = true;
-    }
-  }
-  if (!chunked) {
-    if (T.C == 4) go(k_lines_adj<4, 16, Prob>, 16);
-    else go(k_lines_adj<8, 16, Prob>, 16);
+  if constexpr (XI) {
+    if (T.C == 4) go(k_lines_adj<4, 16, true, Prob>, 16);
+    else go(k_lines_adj<8, 8, true, Prob>, 8);
+  } else {
+    if (T.C == 4) go(k_lines_adj<4, 16, false, Prob>, 16);
+    else go(k_lines_adj<8, 8, false, Prob>, 8);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -1285,6 +1349,12 @@ int launch_lines_adj(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
     return EMX_ERR_HIP;
   }
   return EMX_OK;
+}
+
+template <class Prob>
+int launch_lines_adj(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
+  return dir == 0 ? launch_lines_adj_as<true>(ctx, dir, prob, ih)
+                  : launch_lines_adj_as<false>(ctx, dir, prob, ih);
 }
 
 // Valid chunk sizes per kind.

@@ -7,10 +7,55 @@
 
 namespace emx {
 
-static __global__ void k_zero(double* a, long long n) {
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-       p += (long long)gridDim.x * blockDim.x)
-    a[p] = 0.0;
+// C adjacent values at f, which need not be aligned beyond a double.
+typedef double f64x2u __attribute__((__vector_size__(16), __aligned__(8)));
+template <int C>
+__device__ __forceinline__ void read_w(const double* f, double* v) {
+#pragma unroll
+  for (int i = 0; i < C; i += 2) {
+    const f64x2u t = *reinterpret_cast<const f64x2u*>(f + i);
+    v[i] = t[0];
+    v[i + 1] = t[1];
+  }
+}
+template <int C>
+__device__ __forceinline__ void write_w(double* f, const double* v) {
+#pragma unroll
+  for (int i = 0; i < C; i += 2) *reinterpret_cast<f64x2u*>(f + i) = f64x2u{v[i], v[i + 1]};
+}
+
+// Stores the first m of a chunk's C points (stride st) of one field; with
+// add the old values, all read before the first write, are added to.
+template <int C, bool XI>
+__device__ __forceinline__ void put_chunk(double* f, long long st, int m, double* v, bool add) {
+  if (XI && m == C) {
+    if (add) {
+      double o[C];
+      read_w<C>(f, o);
+#pragma unroll
+      for (int i = 0; i < C; i++) v[i] = o[i] + v[i];
+    }
+    write_w<C>(f, v);
+    return;
+  }
+  if (add) {
+    double o[C];
+#pragma unroll
+    for (int i = 0; i < C; i++) o[i] = i < m ? f[i * st] : 0.0;
+#pragma unroll
+    for (int i = 0; i < C; i++) v[i] = o[i] + v[i];
+  }
+#pragma unroll
+  for (int i = 0; i < C; i++)
+    if (i < m) f[i * st] = v[i];
+}
+
+// Calls f(q, point) for the first m of a chunk's C points.
+template <int C, class F>
+__device__ __forceinline__ void each_point(long long p, long long st, int m, F f) {
+#pragma unroll
+  for (int q = 0; q < C; q++)
+    if (q < m) f(q, p + q * st);
 }
 
 // NV fields, each through D^T along the pass direction; with accumulate
@@ -27,9 +72,26 @@ struct ProbDerivAdj {
 #pragma unroll
     for (int a = 0; a < N_; a++) v[a] = in[a][p];
   }
-  __device__ __forceinline__ void store(long long p, const double* v) const {
+  template <int C>
+  __device__ __forceinline__ void load_w(long long p, double (*v)[NV]) const {
 #pragma unroll
-    for (int a = 0; a < N_; a++) out[a][p] = accumulate ? out[a][p] + v[a] : v[a];
+    for (int a = 0; a < N_; a++) {
+      double t[C];
+      read_w<C>(in[a] + p, t);
+#pragma unroll
+      for (int i = 0; i < C; i++) v[i][a] = t[i];
+    }
+  }
+  template <int C, bool XI>
+  __device__ __forceinline__ void store(long long p, long long st, int m,
+                                        const double (*v)[NV]) const {
+#pragma unroll
+    for (int a = 0; a < N_; a++) {
+      double t[C];
+#pragma unroll
+      for (int i = 0; i < C; i++) t[i] = v[i][a];
+      put_chunk<C, XI>(out[a] + p, st, m, t, accumulate);
+    }
   }
 };
 
@@ -51,264 +113,241 @@ struct ProbDivAdj {
     v[0] = ij * rs_bar[p];
     v[1] = ij * rsv_bar[p];
   }
-  __device__ __forceinline__ void store(long long p, const double* v) const {
-    const double jm = jbn[9 * N + p] * jbn[(4 * dir) * N + p];
-    flux_bar[dir * N + p] = jm * v[0];
-    flux_bar[(3 + dir) * N + p] = jm * v[1];
+  template <int C>
+  __device__ __forceinline__ void load_w(long long p, double (*v)[NV]) const {
+#pragma unroll
+    for (int i = 0; i < C; i++) load(p + i, v[i]);
+  }
+  template <int C, bool XI>
+  __device__ __forceinline__ void store(long long p0, long long st, int m,
+                                        const double (*v)[NV]) const {
+    each_point<C>(p0, st, m, [&](int q, long long p) {
+      const double jm = jbn[9 * N + p] * jbn[(4 * dir) * N + p];
+      flux_bar[dir * N + p] = jm * v[q][0];
+      flux_bar[(3 + dir) * N + p] = jm * v[q][1];
+    });
   }
 };
 
 // Transpose of the linearisation of the five-equation flux divergence
 // (flujos_compact.f90:20-217 fluxes, divergencia.f90 projection) about
-// (um, u, vis, dvel); pres enters linearly, jbn is fixed.  Pass dir forms
-// the eight flux adjoints along dir (convective of 1..5, viscous of 2..4)
-// and scatters them to the input adjoints:
+// (um, u, vis, dvel); pres enters linearly, jbn is fixed.  With
+// x_d[k] = D_d^T(r_k / J) for the eight adjoints r (convective equations
+// 1..5, viscous 2..4), the flux adjoints of direction d are e_d = J m_d x_d,
+// and they scatter to the input adjoints:
 //   conv 1   e = -um(2+d)                 -> um(2+d)
 //   conv 2-4 e = -um(2+d) u(a+1) [-pres]  -> um(2+d), u(a+1), pres (a = d)
 //   conv 5   e = -u(1+d) um5              -> u(1+d), um5
 //   visc a=d  mu*2*(J m_a D_a)            -> vis, dvel(1+4a)
 //   visc a!=d mu*(J_x D_y + J_z D_w)      -> vis, two dvel
-// Pass 0 writes each adjoint, later passes add, except the dvel
-// components a pass touches first (first[] below).
-struct ProbDivAllAdj {
-  static constexpr int NV = 8;
-  static const char* label() { return "flux_div_all_adj"; }
-  double bytes_pt() const {
-    // loads: 8 adjoint fields + 1/J; primal: J, um(2+d), u(1..3), um5,
-    // vis, jbn 1/5/9, five dvel; writes: um(2+d), u(1..3), um5, pres, vis,
-    // five dvel; read back in later passes: u(1..3), um5, pres, vis and
-    // the dvel components touched before
-    const int rmw = pass == 0 ? 0 : 6 + (pass == 1 ? 2 : 4);
-    return 8.0 * (9 + 10 + 5 + 12 + rmw);
-  }
-  FluxIn in;
-  const double* rs_bar;   // 5 fields
-  const double* rsv_bar;  // 5 fields (2..4 used)
-  double* um_bar;         // 5 fields (1 is zero)
-  double* u_bar;          // 3 fields
+// The xi and eta passes only solve: x_0 and x_1 go into the output arrays
+// (slot() below), which the two zeta passes (convective, viscous) read at
+// the points they overwrite with the results of all three directions.  One
+// pass per direction that scattered at once read the primal fields three
+// times and added to its outputs in memory: 1008 B per point and 3 x 236 us
+// at 128^3, against 848 B and 102 + 97 + 148 + 141 us now (4.1 TB/s in the
+// scatter passes, whose registers leave two workgroups on a CU).
+struct AdjScratch {
+  double* um_bar;    // 5 fields (1 is zero)
+  double* u_bar;     // 3 fields
   double* pres_bar;
   double* vis_bar;
-  double* dvel_bar;       // 9 fields
-  int dir, pass;
+  double* dvel_bar;  // 9 fields
+  long long N;
+  // Where x_d[k] is kept, d = 0, 1.  The convective pass overwrites um_bar,
+  // u_bar and pres_bar, the viscous one, which runs after it, the rest.
+  __host__ __device__ __forceinline__ double* slot(int d, int k) const {
+    if (k >= 5) return dvel_bar + (3 * d + k - 5) * N;
+    if (d == 0) return um_bar + k * N;
+    return k < 3 ? u_bar + k * N : (k == 3 ? pres_bar : dvel_bar + 6 * N);
+  }
+};
+
+// The eight solves of the xi or eta pass, four fields to a work-item (all
+// eight: 116-128 us a pass, with half the wavefronts).
+struct ProbDivAllSolve {
+  struct Part {
+    static constexpr int NV = 4;
+    const double* in[4];
+    double* out[4];
+    const double* ij;
+    __device__ __forceinline__ void load(long long p, double* v) const {
+      const double j = ij[p];
+#pragma unroll
+      for (int a = 0; a < 4; a++) v[a] = j * in[a][p];
+    }
+    template <int C>
+    __device__ __forceinline__ void load_w(long long p, double (*v)[NV]) const {
+      double j[C];
+      read_w<C>(ij + p, j);
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        double t[C];
+        read_w<C>(in[a] + p, t);
+#pragma unroll
+        for (int i = 0; i < C; i++) v[i][a] = j[i] * t[i];
+      }
+    }
+    template <int C, bool XI>
+    __device__ __forceinline__ void store(long long p, long long st, int m,
+                                          const double (*v)[NV]) const {
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        double t[C];
+#pragma unroll
+        for (int i = 0; i < C; i++) t[i] = v[i][a];
+        put_chunk<C, XI>(out[a] + p, st, m, t, false);
+      }
+    }
+  };
+  static const char* label() { return "flux_div_all_adj[solve]"; }
+  double bytes_pt() const { return 8.0 * 17; }
+  static constexpr bool INTERLEAVE = true;  // 1/J
+  Part lo, hi;
+  static int parts() { return 2; }
+  __host__ __device__ __forceinline__ Part part(int z) const { return z == 0 ? lo : hi; }
+};
+
+// The convective half of the zeta pass.
+struct ProbDivAllConv {
+  static constexpr int NV = 5;
+  static constexpr int ADJ_WAVES = 4;
+  static const char* label() { return "flux_div_all_adj[conv]"; }
+  // rs_bar and 1/J; x_0, x_1, um 2..5, u, J and three metrics; um_bar,
+  // u_bar, pres_bar
+  double bytes_pt() const { return 8.0 * (6 + 10 + 4 + 3 + 4 + 9); }
+  FluxIn in;
+  const double* rs_bar;
+  AdjScratch o;
   __device__ __forceinline__ void load(long long p, double* v) const {
-    const long long N = in.N;
-    const double ij = in.jbn[10 * N + p];
+    const double ij = in.J(11, p);
 #pragma unroll
-    for (int a = 0; a < 5; a++) v[a] = ij * rs_bar[a * N + p];
-#pragma unroll
-    for (int a = 0; a < 3; a++) v[5 + a] = ij * rsv_bar[(1 + a) * N + p];
+    for (int a = 0; a < 5; a++) v[a] = ij * rs_bar[a * in.N + p];
   }
-  // The scatter of a work-item's W consecutive points p .. p+W-1 of one
-  // line, used where the line is contiguous in memory (the xi pass): in
-  // two phases (convective, viscous), each of which reads all its input
-  // fields for the W points before it computes and writes its outputs, so
-  // every cache line a wavefront touches is used whole by a few consecutive
-  // instructions and the loads of a phase overlap.  (Point by point, each
-  // line of every field was visited once per point, two dozen fields
-  // apart, and was evicted from L2 between the visits.)  Per point the
-  // same arithmetic in the same order as store().
-  static constexpr bool CHUNK_STORE = true;
-  template <int W>
-  __device__ __forceinline__ void putw(double* f, const double* v, bool first) const {
-    if (first) {
+  template <int C, bool XI>
+  __device__ __forceinline__ void store(long long p0, long long st, int m,
+                                        const double (*v)[NV]) const {
+    each_point<C>(p0, st, m, [&](int q, long long p) {
+      const long long N = in.N;
+      double x[3][5], umd[3], u[3];
 #pragma unroll
-      for (int i = 0; i < W; i++) f[i] = v[i];
-    } else {
-      double o[W];
-#pragma unroll
-      for (int i = 0; i < W; i++) o[i] = f[i];
-#pragma unroll
-      for (int i = 0; i < W; i++) f[i] = o[i] + v[i];
-    }
-  }
-  template <int W>
-  __device__ __forceinline__ void store_w(long long p, const double (*x)[NV]) const {
-    const long long N = in.N;
-    const int d = dir;
-    const bool first = pass == 0;
-    const double* jb = in.jbn + p;
-    double jm[W];
-#pragma unroll
-    for (int i = 0; i < W; i++) jm[i] = jb[9 * N + i] * jb[(4 * d) * N + i];
-    // projected flux adjoint k of point i (convective k < 5, viscous 5..7)
-    auto e = [&](int i, int k) { return jm[i] * x[i][k]; };
-    // --- convective: inputs um(2+d), u(1..3), um5 ---
-    {
-      double umd[W], uu[3][W], um5[W];
-#pragma unroll
-      for (int i = 0; i < W; i++) umd[i] = in.um[(1 + d) * N + p + i];
-#pragma unroll
-      for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int i = 0; i < W; i++) uu[a][i] = in.u[a * N + p + i];
-#pragma unroll
-      for (int i = 0; i < W; i++) um5[i] = in.um[4 * N + p + i];
-      double r[W];
-      // um_bar(2+d) = -e1 - sum_a e(2+a) u(1+a): only this pass writes it
-#pragma unroll
-      for (int i = 0; i < W; i++) {
-        double t = -e(i, 0);
-#pragma unroll
-        for (int a = 0; a < 3; a++) t -= e(i, 1 + a) * uu[a][i];
-        r[i] = t;
+      for (int k = 0; k < 5; k++) {
+        x[0][k] = o.slot(0, k)[p];
+        x[1][k] = o.slot(1, k)[p];
+        x[2][k] = v[q][k];
       }
+      const double J = in.J(10, p);
 #pragma unroll
-      for (int i = 0; i < W; i++) um_bar[(1 + d) * N + p + i] = r[i];
+      for (int d = 0; d < 3; d++) {
+        umd[d] = in.UM(2 + d, p);
+        u[d] = in.U(1 + d, p);
+        const double jm = J * in.J(1 + 4 * d, p);
 #pragma unroll
-      for (int a = 0; a < 3; a++) {
+        for (int k = 0; k < 5; k++) x[d][k] = jm * x[d][k];
+      }
+      const double um5 = in.UM(5, p);
+      o.um_bar[p] = 0.0;  // um(1) does not enter any flux
 #pragma unroll
-        for (int i = 0; i < W; i++) {
-          double g = -e(i, 1 + a) * umd[i];
-          if (a == d) g -= e(i, 4) * um5[i];
-          r[i] = g;
+      for (int d = 0; d < 3; d++) {
+        double t = -x[d][0];
+#pragma unroll
+        for (int a = 0; a < 3; a++) t -= x[d][1 + a] * u[a];
+        o.um_bar[(1 + d) * N + p] = t;
+      }
+      double b5 = 0.0, bp = 0.0, bu[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          double g = -x[d][1 + a] * umd[d];
+          if (a == d) g -= x[d][4] * um5;
+          bu[a] = d == 0 ? g : bu[a] + g;
         }
-        putw<W>(u_bar + a * N + p, r, first);
+        b5 = d == 0 ? -x[d][4] * u[d] : b5 + -x[d][4] * u[d];
+        bp = d == 0 ? -x[d][1 + d] : bp + -x[d][1 + d];
       }
-      // u(1+d) by selects (a run-time index would put the arrays in scratch)
+      o.um_bar[4 * N + p] = b5;
 #pragma unroll
-      for (int i = 0; i < W; i++)
-        r[i] = -e(i, 4) * (d == 0 ? uu[0][i] : (d == 1 ? uu[1][i] : uu[2][i]));
-      putw<W>(um_bar + 4 * N + p, r, first);
+      for (int a = 0; a < 3; a++) o.u_bar[a * N + p] = bu[a];
+      o.pres_bar[p] = bp;
+    });
+  }
+};
+
+// The viscous half.
+struct ProbDivAllVisc {
+  static constexpr int NV = 3;
+  static constexpr int ADJ_WAVES = 4;
+  static const char* label() { return "flux_div_all_adj[visc]"; }
+  // rsv_bar 2..4 and 1/J; x_0, x_1, vis, J and three metrics, dvel;
+  // vis_bar, dvel_bar
+  double bytes_pt() const { return 8.0 * (4 + 6 + 1 + 4 + 9 + 10); }
+  FluxIn in;
+  const double* rsv_bar;
+  AdjScratch o;
+  __device__ __forceinline__ void load(long long p, double* v) const {
+    const double ij = in.J(11, p);
 #pragma unroll
-      for (int i = 0; i < W; i++) r[i] = -(d == 0 ? e(i, 1) : (d == 1 ? e(i, 2) : e(i, 3)));
-      putw<W>(pres_bar + p, r, first);
-    }
-    // --- viscous: inputs vis, jbn 1/5/9 and the five dvel components of
-    // this direction; pass that first touches dvel component m (1-based):
-    // 1,2,3,4,7 -> 0; 5,6,8 -> 1; 9 -> 2 ---
-    {
-      // the two (metric, gradient) pairs of viscous flux a != d, and the
-      // diagonal one of a == d (metric jbn 1+4a, gradient 1+4a)
-      auto pair = [&](int a, int& jx, int& mx, int& jz, int& mz) {
-        const int lo = a < d ? a : d, hi = a < d ? d : a;
-        if (lo == 0 && hi == 1) { jx = 1; mx = 2; jz = 5; mz = 4; }       // J1*D2 + J5*D4
-        else if (lo == 0) { jx = 1; mx = 3; jz = 9; mz = 7; }             // J1*D3 + J9*D7
-        else { jx = 9; mx = 8; jz = 5; mz = 6; }                          // J9*D8 + J5*D6
+    for (int a = 0; a < 3; a++) v[a] = ij * rsv_bar[(1 + a) * in.N + p];
+  }
+  template <int C, bool XI>
+  __device__ __forceinline__ void store(long long p0, long long st, int m,
+                                        const double (*v)[NV]) const {
+    each_point<C>(p0, st, m, [&](int q, long long p) {
+      const long long N = in.N;
+      double e[3][3], Jm[3], D[9], b[9];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        e[0][k] = o.slot(0, 5 + k)[p];
+        e[1][k] = o.slot(1, 5 + k)[p];
+        e[2][k] = v[q][k];
+      }
+      const double J = in.J(10, p), mu = in.vis[p];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        Jm[d] = in.J(1 + 4 * d, p);
+        const double jm = J * Jm[d];
+#pragma unroll
+        for (int k = 0; k < 3; k++) e[d][k] = jm * e[d][k];
+      }
+#pragma unroll
+      for (int k = 0; k < 9; k++) D[k] = in.D(1 + k, p);
+      const double J1 = Jm[0], J5 = Jm[1], J9 = Jm[2];
+      double vis = 0.0;
+      bool set[9] = {};  // resolved at compile time
+      auto dput = [&](int k, double w) {
+        b[k - 1] = set[k - 1] ? b[k - 1] + w : w;
+        set[k - 1] = true;
       };
-      double mu[W], J1[W], J5[W], J9[W];
 #pragma unroll
-      for (int i = 0; i < W; i++) mu[i] = in.vis[p + i];
+      for (int d = 0; d < 3; d++) {
+        double vb = 0.0;
 #pragma unroll
-      for (int i = 0; i < W; i++) J1[i] = jb[i];
-#pragma unroll
-      for (int i = 0; i < W; i++) J5[i] = jb[4 * N + i];
-#pragma unroll
-      for (int i = 0; i < W; i++) J9[i] = jb[8 * N + i];
-      // gradient components: Dp[a][0] the diagonal one of a == d, else
-      // Dp[a][0], Dp[a][1] the pair of flux a (indices fixed at compile
-      // time; d only chooses which loads run)
-      double Dp[3][2][W];
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        if (a == d) {
-#pragma unroll
-          for (int i = 0; i < W; i++) Dp[a][0][i] = in.dvel[(4 * a) * N + p + i];
-        } else {
-          int jx, mx, jz, mz;
-          pair(a, jx, mx, jz, mz);
-#pragma unroll
-          for (int i = 0; i < W; i++) Dp[a][0][i] = in.dvel[(mx - 1) * N + p + i];
-#pragma unroll
-          for (int i = 0; i < W; i++) Dp[a][1][i] = in.dvel[(mz - 1) * N + p + i];
-        }
-      }
-      auto Jv = [&](int jc, int i) { return jc == 1 ? J1[i] : (jc == 5 ? J5[i] : J9[i]); };
-      double vb[W], r[W];
-#pragma unroll
-      for (int i = 0; i < W; i++) vb[i] = 0.0;
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        if (a == d) {
-          const int m = 1 + 4 * a, jc = 1 + 4 * a;
-          const int f0 = (m == 5 || m == 6 || m == 8) ? 1 : (m == 9 ? 2 : 0);
-#pragma unroll
-          for (int i = 0; i < W; i++) {
-            const double w = e(i, 5 + a);
-            vb[i] += w * (2.0 * (Jv(jc, i) * Dp[a][0][i]));
-            r[i] = w * mu[i] * 2.0 * Jv(jc, i);
+        for (int a = 0; a < 3; a++) {
+          const double w = e[d][a];
+          if (a == d) {
+            vb += w * (2.0 * (Jm[a] * D[4 * a]));
+            dput(1 + 4 * a, w * mu * 2.0 * Jm[a]);
+          } else if (a + d == 1) {  // J1*D2 + J5*D4
+            vb += w * (J1 * D[1] + J5 * D[3]);
+            dput(2, w * mu * J1);
+            dput(4, w * mu * J5);
+          } else if (a + d == 2) {  // J1*D3 + J9*D7
+            vb += w * (J1 * D[2] + J9 * D[6]);
+            dput(3, w * mu * J1);
+            dput(7, w * mu * J9);
+          } else {                  // J9*D8 + J5*D6
+            vb += w * (J9 * D[7] + J5 * D[5]);
+            dput(8, w * mu * J9);
+            dput(6, w * mu * J5);
           }
-          putw<W>(dvel_bar + (m - 1) * N + p, r, f0 == d);
-        } else {
-          int jx, mx, jz, mz;
-          pair(a, jx, mx, jz, mz);
-#pragma unroll
-          for (int i = 0; i < W; i++)
-            vb[i] += e(i, 5 + a) * (Jv(jx, i) * Dp[a][0][i] + Jv(jz, i) * Dp[a][1][i]);
-          const int fx = (mx == 5 || mx == 6 || mx == 8) ? 1 : (mx == 9 ? 2 : 0);
-          const int fz = (mz == 5 || mz == 6 || mz == 8) ? 1 : (mz == 9 ? 2 : 0);
-#pragma unroll
-          for (int i = 0; i < W; i++) r[i] = e(i, 5 + a) * mu[i] * Jv(jx, i);
-          putw<W>(dvel_bar + (mx - 1) * N + p, r, fx == d);
-#pragma unroll
-          for (int i = 0; i < W; i++) r[i] = e(i, 5 + a) * mu[i] * Jv(jz, i);
-          putw<W>(dvel_bar + (mz - 1) * N + p, r, fz == d);
         }
+        vis = d == 0 ? vb : vis + vb;
       }
-      putw<W>(vis_bar + p, vb, first);
-    }
-  }
-  __device__ __forceinline__ void put(double* f, long long p, double v, bool first) const {
-    f[p] = first ? v : f[p] + v;
-  }
-  __device__ __forceinline__ void store(long long p, const double* x) const {
-    const long long N = in.N;
-    const int d = dir;
-    const bool first = pass == 0;
-    const double jm = in.jbn[9 * N + p] * in.jbn[(4 * d) * N + p];
-    double e[5], ev[3];
+      o.vis_bar[p] = vis;
 #pragma unroll
-    for (int k = 0; k < 5; k++) e[k] = jm * x[k];
-#pragma unroll
-    for (int k = 0; k < 3; k++) ev[k] = jm * x[5 + k];
-    // convective
-    const double umd = in.UM(2 + d, p);
-    double t = -e[0];
-#pragma unroll
-    for (int a = 0; a < 3; a++) t -= e[1 + a] * in.U(1 + a, p);
-    um_bar[(1 + d) * N + p] = t;  // component 2+d: only this pass
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      double g = -e[1 + a] * umd;
-      if (a == d) g -= e[4] * in.UM(5, p);
-      put(u_bar + a * N, p, g, first);
-    }
-    put(um_bar + 4 * N, p, -e[4] * in.U(1 + d, p), first);
-    put(pres_bar, p, -e[1 + d], first);
-    // viscous; pass that first touches dvel component m (1-based):
-    // 1,2,3,4,7 -> 0; 5,6,8 -> 1; 9 -> 2
-    const double mu = in.vis[p];
-    const double J1 = in.J(1, p), J5 = in.J(5, p), J9 = in.J(9, p);
-    auto dput = [&](int m, double v) {
-      const int f0 = (m == 5 || m == 6 || m == 8) ? 1 : (m == 9 ? 2 : 0);
-      put(dvel_bar + (m - 1) * N, p, v, f0 == d);
-    };
-    double vb = 0.0;
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const double w = ev[a];
-      if (a == d) {
-        const int m = 1 + 4 * a;
-        const double Jd = a == 0 ? J1 : (a == 1 ? J5 : J9);
-        vb += w * (2.0 * (Jd * in.D(m, p)));
-        dput(m, w * mu * 2.0 * Jd);
-      } else {
-        const int lo = a < d ? a : d, hi = a < d ? d : a;
-        if (lo == 0 && hi == 1) {  // J1*D2 + J5*D4
-          vb += w * (J1 * in.D(2, p) + J5 * in.D(4, p));
-          dput(2, w * mu * J1);
-          dput(4, w * mu * J5);
-        } else if (lo == 0) {      // J1*D3 + J9*D7
-          vb += w * (J1 * in.D(3, p) + J9 * in.D(7, p));
-          dput(3, w * mu * J1);
-          dput(7, w * mu * J9);
-        } else {                   // J9*D8 + J5*D6
-          vb += w * (J9 * in.D(8, p) + J5 * in.D(6, p));
-          dput(8, w * mu * J9);
-          dput(6, w * mu * J5);
-        }
-      }
-    }
-    put(vis_bar, p, vb, first);
+      for (int k = 0; k < 9; k++) o.dvel_bar[k * N + p] = b[k];
+    });
   }
 };
 
@@ -365,16 +404,19 @@ int op_flux_div_all_adj(emx_ctx* ctx, const double* rs_bar, const double* rsv_ba
   EMX_TRY(adj_ready(ctx));
   const long long N = ctx->d.N();
   const FluxIn in{fp.um, fp.u, nullptr, fp.vis, fp.jbn, fp.dvel, N};
-  for (int d = 0; d < 3; d++) {
-    ProbDivAllAdj p{in, rs_bar, rsv_bar, um_bar, u_bar, pres_bar, vis_bar, dvel_bar, d, d};
+  const AdjScratch o{um_bar, u_bar, pres_bar, vis_bar, dvel_bar, N};
+  for (int d = 0; d < 2; d++) {
+    ProbDivAllSolve p;
+    p.lo.ij = p.hi.ij = fp.jbn + 10 * N;
+    for (int k = 0; k < 8; k++) {
+      ProbDivAllSolve::Part& h = k < 4 ? p.lo : p.hi;
+      h.in[k % 4] = k < 5 ? rs_bar + k * N : rsv_bar + (k - 4) * N;
+      h.out[k % 4] = o.slot(d, k);
+    }
     EMX_TRY(launch_lines_adj(ctx, d, p, ih[d]));
   }
-  // um(1) does not enter any flux
-  EMX_TIMED(ctx, "fill", 8.0 * N,
-            hipLaunchKernelGGL(k_zero, dim3(pointwise_blocks(N)), dim3(256), 0,
-                               ctx->stream, um_bar, N));
-  EMX_TRY_HIP(hipGetLastError());
-  return EMX_OK;
+  EMX_TRY(launch_lines_adj_as<false>(ctx, 2, ProbDivAllConv{in, rs_bar, o}, ih[2]));
+  return launch_lines_adj_as<false>(ctx, 2, ProbDivAllVisc{in, rsv_bar, o}, ih[2]);
 }
 
 }  // namespace emx
