@@ -1,11 +1,11 @@
 // Batched multi-grid stage: many independent grids ("boxes") of uneven
 // sizes advanced together.  One stage = the velocity gradient fused with
 // the velocity divergence (ProbGradDiv, three directional line passes) and
-// one WENO5 / SSP-RK3 level-set step (pad, three stages, the last writing
-// the interior straight into each box's phi).  Every
+// one WENO5 / SSP-RK3 level-set step (three stages, the first reading and
+// the last writing each box's phi itself).  Every
 // phase is ONE launch over all boxes: workgroups are dealt out box by box
 // from per-phase prefix tables (blk_start), each box with its own line
-// tables, geometry and data.  The phase sequence (seven launches) is
+// tables, geometry and data.  The phase sequence (six launches) is
 // captured once in a HIP graph and replayed.  The line-solver shape of
 // each direction (lines per wavefront LG and points per work-item C, i.e.
 // the split between the serial Thomas sweep inside a chunk and the
@@ -109,7 +109,7 @@ struct emx_batch {
   std::vector<Box> box;
   // scratch
   double* acc = nullptr;        // sum of N
-  double* ls = nullptr;         // sum of 3 * NG
+  double* ls = nullptr;         // sum of 2 * NG
   std::vector<long long> acc_off, ls_off;
   // line passes, per direction
   emx::BatchShape shape[3];
@@ -124,8 +124,8 @@ struct emx_batch {
   // level-set phases
   std::vector<emx::LsBatchGrid> ls_h;
   emx::LsBatchGrid* ls_d = nullptr;
-  int* blk_pad_d = nullptr;
-  int nblk_pad = 0;
+  int* blk_ls_d[3] = {nullptr, nullptr, nullptr};  // one table per stage
+  int nblk_ls[3] = {0, 0, 0};
   // state
   bool dirty = true;
   hipGraph_t graph = nullptr;
@@ -153,7 +153,7 @@ void free_batch(emx_batch* b) {
   }
   (void)hipFree(b->waves_d);
   (void)hipFree(b->ls_d);
-  (void)hipFree(b->blk_pad_d);
+  for (int s = 0; s < 3; s++) (void)hipFree(b->blk_ls_d[s]);
   if (b->ev_in) (void)hipEventDestroy(b->ev_in);
   if (b->ev_out) (void)hipEventDestroy(b->ev_out);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -285,7 +285,7 @@ int launch_pass(emx_batch* b, int dir) {
 
 int launch_stage(emx_batch* b) {
   for (int d = 0; d < 3; d++) EMX_TRY(launch_pass(b, d));
-  return op_batch_ls_step(b->stream, b->ls_d, b->blk_pad_d, b->nblk_pad, b->nbox);
+  return op_batch_ls_step(b->stream, b->ls_d, b->blk_ls_d, b->nblk_ls, b->nbox);
 }
 
 // Descriptors of every phase from the bound boxes.
@@ -297,7 +297,6 @@ int commit(emx_batch* b) {
     }
   EMX_TRY(quiesce(b));
   for (int d = 0; d < 3; d++) EMX_TRY(plan_lines(b, d, b->shape[d]));
-  std::vector<int> bp(b->nbox + 1, 0);
   b->ls_h.resize(b->nbox);
   for (int i = 0; i < b->nbox; i++) {
     const Dims& d = b->dims[i];
@@ -311,19 +310,22 @@ int commit(emx_batch* b) {
     G.phi = B.phi;
     G.vel = B.u;
     G.jbn = B.jbn;
-    G.P = base;
-    G.T1 = base + NG;
-    G.T2 = base + 2 * NG;
+    G.T1 = base;
+    G.T2 = base + NG;
     G.iX = 1.0 / B.dxyz[0];
     G.iY = 1.0 / B.dxyz[1];
     G.iZ = 1.0 / B.dxyz[2];
     G.dt = B.dt;
-    bp[i + 1] = bp[i] + (int)((NG + 255) / 256);
   }
-  b->nblk_pad = bp[b->nbox];
+  std::vector<int> blk[3];
+  plan_batch_ls(b->ls_h, blk);
   EMX_TRY_HIP(hipMemcpy(b->ls_d, b->ls_h.data(), b->nbox * sizeof(LsBatchGrid),
                         hipMemcpyHostToDevice));
-  EMX_TRY_HIP(hipMemcpy(b->blk_pad_d, bp.data(), bp.size() * sizeof(int), hipMemcpyHostToDevice));
+  for (int s = 0; s < 3; s++) {
+    b->nblk_ls[s] = blk[s][b->nbox];
+    EMX_TRY_HIP(hipMemcpy(b->blk_ls_d[s], blk[s].data(), blk[s].size() * sizeof(int),
+                          hipMemcpyHostToDevice));
+  }
   EMX_TRY_HIP(hipStreamSynchronize(b->stream));
   b->dirty = false;
   return EMX_OK;
@@ -364,7 +366,7 @@ int emx_batch_create(emx_batch** out, int nbox, const int* dims, int scheme, voi
     b->acc_off.push_back(accN);
     b->ls_off.push_back(lsN);
     accN += d.N();
-    lsN += 3 * emx::ls_padded_points(d.nx, d.ny, d.nz);
+    lsN += 2 * emx::ls_padded_points(d.nx, d.ny, d.nz);
   }
   b->box.resize(nbox);
   if (hipGetDevice(&b->device) != hipSuccess ||
@@ -378,13 +380,13 @@ int emx_batch_create(emx_batch** out, int nbox, const int* dims, int scheme, voi
   bool ok = hipMalloc(&b->acc, accN * sizeof(double)) == hipSuccess &&
             hipMalloc(&b->ls, lsN * sizeof(double)) == hipSuccess &&
             hipMalloc(&b->ls_d, nbox * sizeof(emx::LsBatchGrid)) == hipSuccess &&
-            hipMalloc(&b->blk_pad_d, (nbox + 1) * sizeof(int)) == hipSuccess &&
             hipMalloc(&b->waves_d, nbox * sizeof(emx::BatchWaveLines<emx::ProbGradDiv>)) ==
                 hipSuccess;
   for (int d = 0; d < 3 && ok; d++)
     ok = hipMalloc(&b->lines_d[d], nbox * sizeof(emx::BatchLines<emx::ProbGradDiv>)) ==
              hipSuccess &&
-         hipMalloc(&b->blk_d[d], (nbox + 1) * sizeof(int)) == hipSuccess;
+         hipMalloc(&b->blk_d[d], (nbox + 1) * sizeof(int)) == hipSuccess &&
+         hipMalloc(&b->blk_ls_d[d], (nbox + 1) * sizeof(int)) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     set_error("emx_batch_create: device allocation failed (%lld + %lld doubles)", accN, lsN);

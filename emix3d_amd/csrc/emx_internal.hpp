@@ -58,6 +58,14 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
   return b < 8 * q ? (b % 8) * q + b / 8 : b;
 }
 
+// Workgroup barrier that orders LDS traffic only: global loads issued
+// before it stay in flight (a full __syncthreads also waits for them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Kinds of line solver launch (see compact.hpp).
 enum LineKind {
   KIND_WAVE = 0,       // one wavefront per line, lanes along the line

@@ -321,174 +321,6 @@ __device__ __forceinline__ double bdiff(const double* phi, PDims g, int ax,
   return ih * (gref(phi + id) - gref(phi + id - sxy));
 }
 
-// The backward differences (Dev1thO_Downwind, lsTools.cu:53-95) times the
-// metric m along axis c at offsets -2..+3 from padded point uid (axis
-// position q of n, index stride `stride`).  phi is read once at each of the
-// seven positions q-3..q+3, clamped into the grid (a clamped position's
-// difference is never used by the stencils below); at position 0 the
-// difference is the forward one, phi(1) - phi(0), which is the backward
-// difference at position 1.  Indices are 32-bit: the padded grid has fewer
-// than 2^32 points, so the wrapped unsigned sum is the exact index.
-__device__ __forceinline__ void axis_bd(const double* src, unsigned stride, int q, int n,
-                                        unsigned uid, double ihc, double m, double bd[6]) {
-#pragma clang fp contract(fast)
-  double s[7];
-#pragma unroll
-  for (int o = 0; o < 7; o++) {
-    int t = q - 3 + o;
-    t = t < 0 ? 0 : (t > n - 1 ? n - 1 : t);
-    s[o] = gref(src + (uid + (unsigned)(t - q) * stride));
-  }
-#pragma unroll
-  for (int o = 0; o < 6; o++) bd[o] = ihc * (s[o + 1] - s[o]) * m;
-  if (q == 0) bd[2] = bd[3];
-  if (q == 1) bd[1] = bd[2];
-  if (q == 2) bd[0] = bd[1];
-}
-
-// axis_bd for an axis position q with 3 <= q <= n - 4: every stencil
-// position lies inside the grid, so no clamps and no edge rules.
-__device__ __forceinline__ void axis_bd_inner(const double* src, unsigned stride,
-                                              unsigned uid, double ihc, double m,
-                                              double bd[6]) {
-#pragma clang fp contract(fast)
-  // signed offsets from the point itself: on the x axis (stride 1) they
-  // become the loads' immediate offsets
-  const double* c0 = src + uid;
-  const int st = (int)stride;
-  double s[7];
-#pragma unroll
-  for (int o = 0; o < 7; o++) s[o] = gref(c0 + (o - 3) * st);
-#pragma unroll
-  for (int o = 0; o < 6; o++) bd[o] = ihc * (s[o + 1] - s[o]) * m;
-}
-
-// The five WENO5 operands of the left-biased side along axis c from bd
-// (PhiDevPlusParameterJB, lsTools.cu:587-673: positions q-2..q+2), with the
-// reference's substitutions at the edges.  On the z axis the last plane's
-// fifth operand is the z difference one row down (id_kp2 = id_jm1,
-// lsTools.cu:636).
-__device__ __forceinline__ void stencil_left(const double* src, PDims g, int c, int q, int n,
-                                             int x, int y, int z, double ihc, double m,
-                                             const double bd[6], double b[5]) {
-#pragma unroll
-  for (int t = 0; t < 5; t++) b[t] = bd[t];
-  if (q == 0) { b[1] = bd[2]; b[0] = bd[3]; }
-  if (q == 1) b[0] = bd[1];
-  if (q == n - 2) b[4] = bd[3];
-  if (q == n - 1) {
-    b[3] = bd[2];
-    if (c < 2) b[4] = bd[1];
-    else b[4] = bdiff(src, g, 2, x, y == 0 ? y : y - 1, z, ihc) * m;
-  }
-}
-
-// The right-biased side (PhiDevMinusParameterJB, lsTools.cu:676-770:
-// positions q+3, q+2, q+1, q, q-1) with its edge substitutions.
-__device__ __forceinline__ void stencil_right(int q, int n, const double bd[6], double b[5]) {
-#pragma unroll
-  for (int t = 0; t < 5; t++) b[t] = bd[5 - t];
-  if (q == 0) b[4] = bd[2];
-  if (q == n - 1) { b[2] = bd[2]; b[1] = bd[1]; b[0] = bd[0]; }
-  if (q == n - 2) { b[1] = bd[3]; b[0] = bd[2]; }
-  if (q == n - 3) b[0] = bd[4];
-}
-
-// One fused SSP-RK3 stage of cuAdvectLsJB (lsTransportEc.cu:243-399):
-// backward differences, the upwind JB WENO derivative, the right-hand side
-// advect_RS_WENO (:361-417) and the stage update.  src is the stage input,
-// P the step's initial phi; the stage writes out at every padded point, or,
-// given phi_int (the last stage), only the interior points, straight into
-// the unpadded phi (the values the reference's cuSwapFromGhost copies
-// back).  vel is the interior velocity (3 components of
-// (nx, ny, nz)).  cuAdvectLsJB takes an already padded velocity from a
-// caller the reference does not have, so its ghost values are this
-// library's choice: the even mirror image of the interior for every
-// component (as phi is padded), read at the mirrored coordinates of the
-// interior point instead of from a padded copy.  Near the faces the
-// advected phi therefore follows that choice (an odd reflection of the
-// wall-normal component would be as plausible for a wall); the reference
-// does not pin it.  The metrics (jbn, 11 components of the interior grid;
-// 1, 5, 9 used) are read the same way.
-__device__ __forceinline__ void weno_stage_point(int stage, const double* src,
-                                                 const double* P, const double* vel,
-                                                 const double* jbn, PDims g, double iX,
-                                                 double iY, double iZ, double dt,
-                                                 double* out, double* phi_int, long long id) {
-#pragma clang fp contract(fast)
-  const unsigned uid = (unsigned)id, row = uid / (unsigned)g.x;  // NG < 2^32
-  const int x = (int)(uid - row * (unsigned)g.x), y = (int)(row % (unsigned)g.y),
-            z = (int)(row / (unsigned)g.y);
-  if (phi_int && (x < GC || x >= g.x - GC || y < GC || y >= g.y - GC || z < GC ||
-                  z >= g.z - GC))
-    return;  // a ghost point of the last stage: not part of the result
-  // The last stage reads the second stage's output only within 3 points of
-  // the interior (its stencils' reach), so the second stage skips the two
-  // outermost ghost layers (whose values the reference computes and never
-  // uses for the interior).  The first stage computes every padded point:
-  // the second stage's points reach its outermost layer.
-  constexpr int SKIP = GC - 3;
-  if (stage == 1 && (x < SKIP || x >= g.x - SKIP || y < SKIP || y >= g.y - SKIP ||
-                     z < SKIP || z >= g.z - SKIP))
-    return;
-  const double ih[3] = {iX, iY, iZ};
-  const unsigned nx = (unsigned)(g.x - 2 * GC), ny = (unsigned)(g.y - 2 * GC),
-                 nz = (unsigned)(g.z - 2 * GC);
-  const unsigned vid = (unsigned)mirror(x, (int)nx) +
-                       nx * ((unsigned)mirror(y, (int)ny) + ny * (unsigned)mirror(z, (int)nz));
-  const unsigned vN = nx * ny * nz;
-  const double met[3] = {gref(jbn + vid), gref(jbn + (size_t)4 * vN + vid),
-                         gref(jbn + (size_t)8 * vN + vid)};
-  double r[3];
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    // upwinding (advect_RS_WENO, lsTools.cu:361-417) uses the left-biased
-    // derivative where the velocity is positive and the right-biased one
-    // where it is negative, so only that one is formed:
-    //   0.5(s+1) v L + 0.5|s-1| v R  =  v L (v > 0),  v R (v < 0),  0
-    const double v = gref(vel + (size_t)c * vN + vid);
-    if (v == 0.0) {
-      r[c] = 0.0;
-      continue;
-    }
-    const int pos[3] = {x, y, z}, ext[3] = {g.x, g.y, g.z};
-    const unsigned stride[3] = {1u, (unsigned)g.x, (unsigned)g.x * (unsigned)g.y};
-    double bd[6], b[5];
-    if (pos[c] >= 3 && pos[c] <= ext[c] - 4) {
-      // away from the padded grid's faces: the interior operands, left
-      // (q-2..q+2) or right (q+3..q-1) biased, with no edge rules
-      axis_bd_inner(src, stride[c], uid, ih[c], met[c], bd);
-#pragma unroll
-      for (int t = 0; t < 5; t++) b[t] = v > 0.0 ? bd[t] : bd[5 - t];
-    } else {
-      axis_bd(src, stride[c], pos[c], ext[c], uid, ih[c], met[c], bd);
-      if (v > 0.0) stencil_left(src, g, c, pos[c], ext[c], x, y, z, ih[c], met[c], bd, b);
-      else stencil_right(pos[c], ext[c], bd, b);
-    }
-    r[c] = v * weno5(b[0], b[1], b[2], b[3], b[4]);
-  }
-  const double rs = r[0] + r[1] + r[2];
-  const double sv = gref(src + id);
-  double o;
-  if (stage == 0) o = sv - dt * rs;
-  else if (stage == 1) o = 0.75 * gref(P + id) + 0.25 * (sv - dt * rs);
-  else o = (gref(P + id) + 2.0 * (sv - dt * rs)) * (1.0 / 3.0);
-  if (phi_int)
-    gref(phi_int + ((unsigned)(x - GC) + nx * ((unsigned)(y - GC) + ny * (unsigned)(z - GC)))) = o;
-  else
-    gref(out + id) = o;
-}
-
-__global__ void k_weno_stage(int stage, const double* src, const double* P,
-                             const double* vel, const double* jbn, PDims g,
-                             double iX, double iY, double iZ, double dt,
-                             double* out, double* phi_int) {
-  const long long NG = g.N();
-  for (long long id = (long long)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; id < NG;
-       id += (long long)gridDim.x * blockDim.x)
-    weno_stage_point(stage, src, P, vel, jbn, g, iX, iY, iZ, dt, out, phi_int, id);
-}
-
 // ---------------------------------------------------------------------------
 // Level-set reinitialisation (cuReinitLsJB, lsTransportEc.cu:422-676).
 
@@ -531,9 +363,12 @@ __device__ __forceinline__ double godunov_axis(const double bd[6], double l5) {
   return c;
 }
 
-// The edge rules of axis_bd, stencil_left and stencil_right at position q of
-// n, applied to the six differences: past the low face the first one is
-// repeated, past the high face they are mirrored.
+// The reference's edge rules for the six metric-scaled backward differences
+// bd (offsets -2..+3) of position q of n: the index-0 rule of
+// Dev1thO_Downwind (lsTools.cu:53-95, the forward difference) and the
+// substitutions of PhiDevPlusParameterJB (:587-673, operands bd[0..4]) and
+// PhiDevMinusParameterJB (:676-770, operands bd[5..1]).  Past the low face
+// the first difference is repeated, past the high face they are mirrored.
 __device__ __forceinline__ void edge_bd(double bd[6], int q, int n) {
   if (q == 0) bd[2] = bd[3];
   if (q <= 1) bd[1] = bd[2];
@@ -546,6 +381,49 @@ __device__ __forceinline__ void edge_bd(double bd[6], int q, int n) {
   if (q == n - 3) bd[5] = bd[4];
 }
 
+// The plane of a z-marching workgroup of 256 work-items in LDS: a tile of
+// 2^ltx x 2^(8-ltx) columns (x, y) and three more on either side along each
+// axis (the stencils are along the axes, so no corners), in two buffers taken
+// in turn.  A work-item has its own column's value in registers and loads at
+// most one halo column, so a plane costs two loads per point; read from
+// memory the stencils took 13, and a stage's 19 to 21 loads and stores per
+// point kept the address units 90% busy.
+struct StencilTile {
+  static constexpr int CELLS = 38 * 14;  // 32 x 8; 16 x 16 takes 22 x 22
+  int w, own, halo;  // row stride; cells of the column and of its halo column
+  int hx, hy;        // that column's place in the tile (halo < 0: none)
+  __device__ __forceinline__ StencilTile(int ltx) {
+    const int tx = 1 << ltx, ty = 256 >> ltx;
+    int t = threadIdx.x;
+    w = tx + 6;
+    own = ((t >> ltx) + 3) * w + (t & (tx - 1)) + 3;
+    if (t < 6 * tx) {
+      const int r = t >> ltx;
+      hx = t & (tx - 1);
+      hy = r < 3 ? r - 3 : ty + r - 3;
+    } else {
+      t -= 6 * tx;
+      const int r = t % 6;
+      hx = r < 3 ? r - 3 : tx + r - 3;
+      hy = t / 6;
+    }
+    halo = (int)threadIdx.x < 6 * tx || hy < ty ? (hy + 3) * w + hx + 3 : -1;
+  }
+  __device__ __forceinline__ void put(double* c, double v, double h) const {
+    c[own] = v;
+    if (halo >= 0) c[halo] = h;
+  }
+  // The seven stencil values along x and y around the own column.
+  __device__ __forceinline__ void get(const double* c, double v, double vx[7],
+                                      double vy[7]) const {
+#pragma unroll
+    for (int o = 0; o < 7; o++) {
+      vx[o] = o == 3 ? v : c[own + o - 3];
+      vy[o] = o == 3 ? v : c[own + (o - 3) * w];
+    }
+  }
+};
+
 // One SSP-RK3 stage of the reinitialisation: the two JB WENO derivatives per
 // axis, the Godunov |grad phi| by the sign of phi0 and rs = S(phi0)
 // (|grad phi| - 1), S = phi0/sqrt(phi0^2 + dmin^2) (reini_RS_WENOJB,
@@ -557,40 +435,46 @@ __device__ __forceinline__ void edge_bd(double bd[6], int q, int n) {
 // them), stage 2 the interior points, each written into out, a different
 // array, together with its mirror images in the ghost layers: out is then
 // the next iteration's phi with the ghost mirroring that iteration would
-// start with already applied.
+// start with already applied (given phi, the last iteration, only the
+// interior, into phi).  dmin and jbn (1, 5, 9 used) are interior fields, read
+// at a ghost point's mirror image.
 //
 // A workgroup owns a 32 x 8 tile of (x, y) and marches z through a slab of
-// kz planes with the stencil's z values and differences in registers, so a
-// point loads 13 values of src instead of 21 and the index arithmetic is
-// done once per column.  Bound by instruction issue (about 400 VALU
-// instructions per point-wave, the issue slots 80% busy) with the memory
-// floor (56 B per padded point) close behind: 97 us a stage at 218 x 186 x
-// 170 padded points, 4.1 TB/s, against 182 us for the form with one point
-// per work-item and both WENO derivatives of every axis.  Wider tiles waste
-// lanes at the row ends (64 x 4: 10% slower), 16 x 16 tiles 3%; loading the
-// next plane's streamed fields ahead costs the registers of a fifth
-// wavefront and was 4% slower.  The four fields no stage writes take
-// nontemporal loads, which leaves the last-level cache to phi (1% faster).
+// kz planes with the stencil's z values and differences in registers and the
+// plane in LDS (StencilTile).  At 218 x 186 x 170 padded points a stage takes
+// 94-99 us: 182 us with one point per work-item and both WENO derivatives of
+// every axis, 100-121 us with the x and y stencils read from memory and
+// padded copies of dmin and the metrics (five passes of 28 us a call, now
+// one).  About 400 VALU instructions per point-wave bound it, with the memory
+// floor (24 B per padded and 32 B per interior point) close behind.  Wider
+// tiles waste lanes at the row ends (64 x 4: 10% slower), 16 x 16 tiles 3%.
 constexpr int RI_TX = 32, RI_TY = 8;
 
 template <int STAGE>
 __global__ void __launch_bounds__(256)
-k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const double* j1,
-                  const double* j5, const double* j9, PDims g, int kz, double iX, double iY,
-                  double iZ, double dt, double* out) {
+k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const double* jbn,
+                  PDims g, int kz, double iX, double iY, double iZ, double dt, double* out,
+                  double* phi) {
   constexpr int LO = STAGE == 0 ? 0 : (STAGE == 1 ? GC - 3 : GC);
   const int nbx = (g.x - 2 * LO + RI_TX - 1) / RI_TX, nby = (g.y - 2 * LO + RI_TY - 1) / RI_TY;
   const int b = (int)xcd_block(blockIdx.x, gridDim.x);
-  const int x = LO + (b % nbx) * RI_TX + (int)threadIdx.x % RI_TX;
-  const int y = LO + (b / nbx % nby) * RI_TY + (int)threadIdx.x / RI_TX;
+  const int x0 = LO + (b % nbx) * RI_TX, y0 = LO + (b / nbx % nby) * RI_TY;
+  const int x = x0 + (int)threadIdx.x % RI_TX, y = y0 + (int)threadIdx.x / RI_TX;
   const int z0 = LO + b / (nbx * nby) * kz, z1 = min(z0 + kz, g.z - LO);
   const bool own = x < g.x - LO && y < g.y - LO;
-  // work-items past the tile's end follow the last column and store nothing
-  const int xc = min(x, g.x - 1 - LO), yc = min(y, g.y - 1 - LO);
+  // positions past the padded grid's faces are clamped: work-items there
+  // store nothing, and a difference over one is never used
+  const int xc = min(x, g.x - 1), yc = min(y, g.y - 1);
   const unsigned sy = (unsigned)g.x, sz = (unsigned)g.x * (unsigned)g.y;  // NG < 2^32
   const unsigned col = (unsigned)xc + sy * (unsigned)yc;
-  // stencil positions past the padded grid's faces, clamped (their
-  // differences are never used); none in stage 2
+  const int nx = g.x - 2 * GC, ny = g.y - 2 * GC, nz = g.z - 2 * GC;
+  const unsigned vsz = (unsigned)nx * (unsigned)ny;
+  const size_t vN = (size_t)vsz * (unsigned)nz;
+  const unsigned vcol = (unsigned)mirror(xc, nx) + (unsigned)nx * (unsigned)mirror(yc, ny);
+  __shared__ double cells[2][StencilTile::CELLS];
+  const StencilTile tile(5);
+  const unsigned hcol = (unsigned)min(max(x0 + tile.hx, 0), g.x - 1) +
+                        sy * (unsigned)min(max(y0 + tile.hy, 0), g.y - 1);
   const bool edge_x = STAGE < 2 && __any(xc < 3 || xc > g.x - 4);
   const bool edge_y = STAGE < 2 && __any(yc < 3 || yc > g.y - 4);
   auto clampz = [&](int z) { return STAGE < 2 ? min(max(z, 0), g.z - 1) : z; };
@@ -600,7 +484,6 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
     return reinterpret_cast<const double*>(reinterpret_cast<const char*>(f) + off);
   };
   auto ld = [&](const double* f, unsigned off) { return *at(f, off); };
-  auto ldn = [&](const double* f, unsigned off) { return __builtin_nontemporal_load(at(f, off)); };
   auto plane = [&](int z) { return ld(src, (col + (unsigned)clampz(z) * sz) * 8u); };
   double vz[4], dz[6];  // values of planes z .. z+3; the stencil's differences along z
 #pragma unroll
@@ -613,6 +496,7 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
     dz[4] = vz[2] - vz[1];
     dz[5] = vz[3] - vz[2];
   }
+  double hv = ld(src, (hcol + (unsigned)z0 * sz) * 8u);
   for (int z = z0; z < z1; z++) {
 #pragma unroll
     for (int o = 0; o < 3; o++) vz[o] = vz[o + 1];
@@ -621,20 +505,14 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
     vz[3] = plane(z + 3);
     dz[5] = vz[3] - vz[2];
     const unsigned id = col + (unsigned)z * sz, off = id * 8u;
+    const unsigned vid = vcol + (unsigned)mirror(z, nz) * vsz, voff = vid * 8u;
     const double sv = vz[0];
     double vx[7], vy[7];
-#pragma unroll
-    for (int o = 0; o < 7; o++) {
-      if (o == 3) vx[o] = vy[o] = sv;
-      else if (edge_x) vx[o] = ld(src, (id + (unsigned)(min(max(xc - 3 + o, 0), g.x - 1) - xc)) * 8u);
-      else vx[o] = ld(src + (o - 3), off);
-    }
-#pragma unroll
-    for (int o = 0; o < 7; o++) {
-      if (o == 3) continue;
-      if (edge_y) vy[o] = ld(src, (id + (unsigned)(min(max(yc - 3 + o, 0), g.y - 1) - yc) * sy) * 8u);
-      else vy[o] = ld(src + (o - 3) * (int)sy, off);
-    }
+    double* c = cells[(z - z0) & 1];
+    tile.put(c, sv, hv);
+    lds_barrier();
+    if (z + 1 < z1) hv = ld(src, (hcol + (unsigned)(z + 1) * sz) * 8u);
+    tile.get(c, sv, vx, vy);
     const double p0 = STAGE == 0 ? sv : ld(P, off);
     // metric / spacing with the sign of phi0 (at phi0 = 0, S and with it rs
     // vanish)
@@ -642,8 +520,9 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
       return __longlong_as_double(__double_as_longlong(s) ^
                                   (__double_as_longlong(p0) & (long long)(1ull << 63)));
     };
-    const double sx = signed_by_p0(iX * ldn(j1, off)), sY = signed_by_p0(iY * ldn(j5, off)),
-                 sZ = signed_by_p0(iZ * ldn(j9, off)), d = ldn(dmin, off);
+    const double sx = signed_by_p0(iX * ld(jbn, voff)),
+                 sY = signed_by_p0(iY * ld(jbn + 4 * vN, voff)),
+                 sZ = signed_by_p0(iZ * ld(jbn + 8 * vN, voff)), d = ld(dmin, voff);
     double bx[6], by[6], bz[6];
 #pragma unroll
     for (int o = 0; o < 6; o++) {
@@ -674,6 +553,10 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
       // (P + 2 step)/3, the quotient corrected by its residual
       const double t = p0 + 2.0 * step, o3 = t * (1.0 / 3.0);
       const double o = __builtin_fma(__builtin_fma(-3.0, o3, t), 1.0 / 3.0, o3);
+      if (phi) {
+        phi[vid] = o;
+        continue;
+      }
       int cx[3], cy[3], cz[3];
       const int kx = mirror_images(x, g.x - 2 * GC, cx), ky = mirror_images(y, g.y - 2 * GC, cy),
                 kk = mirror_images(z, g.z - 2 * GC, cz);
@@ -687,8 +570,8 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
 
 template <int STAGE>
 void launch_reinit_stage(hipStream_t st, const double* src, const double* P, const double* dmin,
-                         const double* j1, const double* j5, const double* j9, PDims g, double iX,
-                         double iY, double iZ, double dt, double* out) {
+                         const double* jbn, PDims g, double iX, double iY, double iZ, double dt,
+                         double* out, double* phi = nullptr) {
   constexpr int LO = STAGE == 0 ? 0 : (STAGE == 1 ? GC - 3 : GC);
   const long long cols = (long long)((g.x - 2 * LO + RI_TX - 1) / RI_TX) *
                          ((g.y - 2 * LO + RI_TY - 1) / RI_TY);
@@ -698,52 +581,202 @@ void launch_reinit_stage(hipStream_t st, const double* src, const double* P, con
   int kz = 8;
   while (kz > 2 && cols * ((nz + kz - 1) / kz) < 1024) kz /= 2;
   hipLaunchKernelGGL(k_ls_reinit_stage<STAGE>, dim3((unsigned)(cols * ((nz + kz - 1) / kz))),
-                     dim3(256), 0, st, src, P, dmin, j1, j5, j9, g, kz, iX, iY, iZ, dt, out);
+                     dim3(256), 0, st, src, P, dmin, jbn, g, kz, iX, iY, iZ, dt, out, phi);
 }
 
 // ---------------------------------------------------------------------------
-// The same step for many grids in one launch per phase (the batched stage):
-// workgroup b serves grid gi with blk_start[gi] <= b < blk_start[gi+1],
-// points (b - blk_start[gi])*256 + threadIdx.x of the padded grid (the pad
-// and the three stages; the last writes the interior of phi).
-__device__ __forceinline__ int batch_grid(const int* blk_start, int ngrid) {
+// Level-set advection (cuAdvectLsJB, lsTransportEc.cu:243-399).
+
+// First point of the range that stage 0, 1, 2 computes in every direction of
+// the padded grid (it ends as far from the other face).  The last stage
+// computes the interior; its stencils reach three points further, so the
+// second stage skips the two outermost ghost layers (whose values the
+// reference computes and never uses for the interior), and that stage's
+// points reach the outermost layer of the first one.
+constexpr int adv_first(int stage) { return stage == 0 ? 0 : (stage == 1 ? GC - 3 : GC); }
+
+// Workgroup tiles of the advection: 2^ltx x 2^(8-ltx) columns (x, y), 32 x 8
+// unless 16 x 16 leaves fewer work-items past the ends of the rows and
+// columns.
+int adv_ltx(const PDims& g) {
+  auto covered = [&](int l) {
+    return (long long)(((g.x + (1 << l) - 1) >> l) << l) *
+           (((g.y + (256 >> l) - 1) >> (8 - l)) << (8 - l));
+  };
+  return covered(4) < covered(5) ? 4 : 5;
+}
+
+// Slabs of 8 planes (16: 3% slower on 48 boxes of 25.7 M points), fewer while
+// the chip's 256 compute units would get less than four workgroups.
+int adv_blocks(const PDims& g, int stage, int ltx, int kz) {
+  const int lo = adv_first(stage);
+  return ((g.x - 2 * lo + (1 << ltx) - 1) >> ltx) *
+         ((g.y - 2 * lo + (256 >> ltx) - 1) >> (8 - ltx)) * ((g.z - 2 * lo + kz - 1) / kz);
+}
+
+// One fused SSP-RK3 stage for the columns of workgroup b of a grid: backward
+// differences, the upwind JB WENO derivative, the right-hand side
+// advect_RS_WENO (lsTools.cu:361-417) and the stage update.  phi, vel (3
+// components) and jbn (11; 1, 5, 9 used) are interior fields, read at a
+// ghost point's mirror image, so the padded copies of the reference are not
+// made: stage 0 takes its stencils straight from phi.  Stages 0 and 1 write
+// the padded arrays T1 and T2 (out), the next stage's src; stage 2 writes
+// phi in place, whose other points it does not read.
+//
+// cuAdvectLsJB takes an already padded velocity from a caller the reference
+// does not have, so its ghost values are this library's choice: the even
+// mirror image of the interior for every component (as phi is padded).  Near
+// the faces the advected phi follows that choice (an odd reflection of the
+// wall-normal component would be as plausible for a wall); the reference
+// does not pin it.
+//
+// The march along z and the derivative are those of k_ls_reinit_stage.  The
+// form with one point per work-item formed every operand from 21 loads and
+// found its place by divisions; with the padded copy of phi it took 162 +
+// 3 x 694 us on 48 boxes of 25.7 M points (36.4 M padded).  Now
+// 497 + 511 + 454 us (3.9 TB/s); 643 + 637 + 498 us with the x and y stencils
+// read from memory instead of StencilTile, and 727 + 728 + 566 us with
+// nontemporal loads of vel and jbn, whose lines neighbouring tiles share.
+template <int STAGE>
+__device__ __forceinline__ void ls_advect_tile(const double* src, const double* phi,
+                                               const double* vel, const double* jbn, PDims g,
+                                               int b, int ltx, int kz, double iX, double iY,
+                                               double iZ, double dt, double* out) {
+#pragma clang fp contract(fast)
+  constexpr int LO = adv_first(STAGE);
+  const int nbx = (g.x - 2 * LO + (1 << ltx) - 1) >> ltx,
+            nby = (g.y - 2 * LO + (256 >> ltx) - 1) >> (8 - ltx);
+  const int x0 = LO + ((b % nbx) << ltx), y0 = LO + ((b / nbx % nby) << (8 - ltx));
+  const int x = x0 + ((int)threadIdx.x & ((1 << ltx) - 1)), y = y0 + ((int)threadIdx.x >> ltx);
+  const int z0 = LO + b / (nbx * nby) * kz, z1 = min(z0 + kz, g.z - LO);
+  const bool own = x < g.x - LO && y < g.y - LO;
+  // positions past the padded grid's faces are clamped: work-items there
+  // store nothing, and a difference over one is never used
+  const int xc = min(x, g.x - 1), yc = min(y, g.y - 1);
+  const int nx = g.x - 2 * GC, ny = g.y - 2 * GC, nz = g.z - 2 * GC;
+  const unsigned vsz = (unsigned)nx * (unsigned)ny;
+  const size_t vN = (size_t)vsz * (unsigned)nz;
+  const unsigned vcol = (unsigned)mirror(xc, nx) + (unsigned)nx * (unsigned)mirror(yc, ny);
+  // src: the padded grid, or phi through the mirror images
+  const unsigned sy = STAGE == 0 ? (unsigned)nx : (unsigned)g.x;
+  const unsigned sz = STAGE == 0 ? vsz : (unsigned)g.x * (unsigned)g.y;
+  auto place = [&](int t, int gn, int n) {
+    t = min(max(t, 0), gn - 1);
+    return (unsigned)(STAGE == 0 ? mirror(t, n) : t);
+  };
+  const unsigned col = place(xc, g.x, nx) + sy * place(yc, g.y, ny);
+  __shared__ double cells[2][StencilTile::CELLS];
+  const StencilTile tile(ltx);
+  const unsigned hcol = place(x0 + tile.hx, g.x, nx) + sy * place(y0 + tile.hy, g.y, ny);
+  const bool edge_x = STAGE < 2 && __any(xc < 3 || xc > g.x - 4);
+  const bool edge_y = STAGE < 2 && __any(yc < 3 || yc > g.y - 4);
+  // a field's value at byte offset off (the padded grid has fewer than 2^29
+  // points): uniform base, 32-bit offset
+  auto at = [](const double* f, unsigned off) -> decltype(auto) {
+    return gref(reinterpret_cast<const double*>(reinterpret_cast<const char*>(f) + off));
+  };
+  auto ld = [&](const double* f, unsigned off) -> double { return at(f, off); };
+  auto plane_of = [&](unsigned c, int z) { return ld(src, (c + place(z, g.z, nz) * sz) * 8u); };
+  auto plane = [&](int z) { return plane_of(col, z); };
+  double vz[4], dz[6];  // values of planes z .. z+3; the stencil's differences along z
+#pragma unroll
+  for (int o = 0; o < 3; o++) vz[o + 1] = plane(z0 + o);
+  {
+    const double a = plane(z0 - 3), b2 = plane(z0 - 2), c = plane(z0 - 1);
+    dz[1] = b2 - a;
+    dz[2] = c - b2;
+    dz[3] = vz[1] - c;
+    dz[4] = vz[2] - vz[1];
+    dz[5] = vz[3] - vz[2];
+  }
+  double hv = plane_of(hcol, z0);
+  for (int z = z0; z < z1; z++) {
+#pragma unroll
+    for (int o = 0; o < 3; o++) vz[o] = vz[o + 1];
+#pragma unroll
+    for (int o = 0; o < 5; o++) dz[o] = dz[o + 1];
+    vz[3] = plane(z + 3);
+    dz[5] = vz[3] - vz[2];
+    const unsigned voff = (vcol + (unsigned)mirror(z, nz) * vsz) * 8u;
+    const double sv = vz[0];
+    double vx[7], vy[7];
+    double* c = cells[(z - z0) & 1];
+    tile.put(c, sv, hv);
+    lds_barrier();
+    if (z + 1 < z1) hv = plane_of(hcol, z + 1);
+    tile.get(c, sv, vx, vy);
+    const double p0 = STAGE == 0 ? sv : ld(phi, voff);
+    // upwinding: the left-biased derivative where the velocity is positive
+    // and the right-biased one where it is negative, so only that one is
+    // formed: 0.5(s+1) v L + 0.5|s-1| v R  =  v L (v > 0),  v R (v < 0),  0
+    auto axis = [&](double v, const double bd[6], double l5) {
+      const bool left = v > 0.0;
+      const double b1 = left ? bd[0] : bd[5], b2 = left ? bd[1] : bd[4],
+                   b3 = left ? bd[2] : bd[3], b4 = left ? bd[3] : bd[2], b5 = left ? l5 : bd[1];
+      return v == 0.0 ? 0.0 : v * weno5(b1, b2, b3, b4, b5);
+    };
+    double bd[6];
+    const double mx = iX * ld(jbn, voff), mY = iY * ld(jbn + 4 * vN, voff),
+                 mZ = iZ * ld(jbn + 8 * vN, voff);
+    const double ux = ld(vel, voff), uy = ld(vel + vN, voff), uz = ld(vel + 2 * vN, voff);
+#pragma unroll
+    for (int o = 0; o < 6; o++) bd[o] = mx * (vx[o + 1] - vx[o]);
+    if (edge_x) edge_bd(bd, xc, g.x);
+    double rs = axis(ux, bd, bd[4]);
+#pragma unroll
+    for (int o = 0; o < 6; o++) bd[o] = mY * (vy[o + 1] - vy[o]);
+    if (edge_y) edge_bd(bd, yc, g.y);
+    rs += axis(uy, bd, bd[4]);
+#pragma unroll
+    for (int o = 0; o < 6; o++) bd[o] = mZ * dz[o];
+    double z5 = bd[4];
+    if (STAGE < 2 && (z < 3 || z > g.z - 4)) {
+      edge_bd(bd, z, g.z);
+      z5 = bd[4];
+      if (z == g.z - 1) {
+        // on the last plane L's fifth operand is the z difference one row
+        // down (id_kp2 = id_jm1, lsTools.cu:636)
+        const unsigned row = place(xc, g.x, nx) + sy * place(yc == 0 ? 0 : yc - 1, g.y, ny);
+        z5 = mZ * (plane_of(row, z) - plane_of(row, z - 1));
+      }
+    }
+    rs += axis(uz, bd, z5);
+    if (!own) continue;
+    double o;
+    if (STAGE == 0) o = sv - dt * rs;
+    else if (STAGE == 1) o = 0.75 * p0 + 0.25 * (sv - dt * rs);
+    else o = (p0 + 2.0 * (sv - dt * rs)) * (1.0 / 3.0);
+    gref(out + (STAGE == 2 ? vcol + (unsigned)(z - GC) * vsz
+                           : (unsigned)xc + (unsigned)g.x *
+                                 ((unsigned)yc + (unsigned)g.y * (unsigned)z))) = o;
+  }
+}
+
+template <int STAGE>
+__global__ void __launch_bounds__(256)
+k_ls_advect(const double* src, const double* phi, const double* vel, const double* jbn, PDims g,
+            int ltx, int kz, double iX, double iY, double iZ, double dt, double* out) {
+  ls_advect_tile<STAGE>(src, phi, vel, jbn, g, (int)xcd_block(blockIdx.x, gridDim.x), ltx, kz, iX,
+                        iY, iZ, dt, out);
+}
+
+// The same for many grids in one launch (the batched stage): workgroup b
+// serves grid gi with blk_start[gi] <= b < blk_start[gi+1].
+template <int STAGE>
+__global__ void __launch_bounds__(256)
+k_batch_advect(const LsBatchGrid* grids, const int* blk_start, int ngrid) {
   const int b = (int)xcd_block(blockIdx.x, gridDim.x);
-  int lo = 0, hi = ngrid;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (blk_start[mid] <= b) lo = mid;
+  int gi = 0, hi = ngrid;
+  while (hi - gi > 1) {
+    const int mid = (gi + hi) >> 1;
+    if (blk_start[mid] <= b) gi = mid;
     else hi = mid;
   }
-  return lo;
-}
-
-__global__ void __launch_bounds__(256)
-k_batch_pad(const LsBatchGrid* grids, const int* blk_start, int ngrid) {
-  const int gi = batch_grid(blk_start, ngrid);
   const LsBatchGrid& G = grids[gi];
   const PDims g{G.nx + 2 * GC, G.ny + 2 * GC, G.nz + 2 * GC};
-  const long long p = (long long)((int)xcd_block(blockIdx.x, gridDim.x) - blk_start[gi]) * 256 + threadIdx.x;
-  if (p >= g.N()) return;
-  const unsigned up = (unsigned)p, row = up / (unsigned)g.x;
-  const int i = (int)(up - row * (unsigned)g.x), j = (int)(row % (unsigned)g.y),
-            k = (int)(row / (unsigned)g.y);
-  const long long src = mirror(i, G.nx) + (long long)G.nx * (mirror(j, G.ny) +
-                                                             (long long)G.ny * mirror(k, G.nz));
-  gref(G.P + p) = gref(G.phi + src);
-}
-
-__global__ void __launch_bounds__(256)
-k_batch_weno_stage(const LsBatchGrid* grids, const int* blk_start, int ngrid, int stage) {
-  const int gi = batch_grid(blk_start, ngrid);
-  const LsBatchGrid& G = grids[gi];
-  const PDims g{G.nx + 2 * GC, G.ny + 2 * GC, G.nz + 2 * GC};
-  const long long NG = g.N();
-  const long long id = (long long)((int)xcd_block(blockIdx.x, gridDim.x) - blk_start[gi]) * 256 + threadIdx.x;
-  if (id >= NG) return;
-  const double* src = stage == 0 ? G.P : (stage == 1 ? G.T1 : G.T2);
-  double* out = stage == 0 ? G.T1 : G.T2;
-  weno_stage_point(stage, src, G.P, G.vel, G.jbn, g, G.iX, G.iY, G.iZ,
-                   G.dt, out, stage == 2 ? G.phi : nullptr, id);
+  ls_advect_tile<STAGE>(STAGE == 0 ? G.phi : (STAGE == 1 ? G.T1 : G.T2), G.phi, G.vel, G.jbn, g,
+                        b - blk_start[gi], G.ltx, G.kz, G.iX, G.iY, G.iZ, G.dt,
+                        STAGE == 0 ? G.T1 : (STAGE == 1 ? G.T2 : G.phi));
 }
 
 unsigned blocks_for(long long n) {
@@ -768,12 +801,34 @@ long long ls_padded_points(int nx, int ny, int nz) {
   return (long long)(nx + 2 * GC) * (ny + 2 * GC) * (nz + 2 * GC);
 }
 
-int op_batch_ls_step(hipStream_t st, const LsBatchGrid* grids, const int* blk_pad,
-                     int nblk_pad, int ngrid) {
-  hipLaunchKernelGGL(k_batch_pad, dim3(nblk_pad), dim3(256), 0, st, grids, blk_pad, ngrid);
-  for (int stage = 0; stage < 3; stage++)
-    hipLaunchKernelGGL(k_batch_weno_stage, dim3(nblk_pad), dim3(256), 0, st, grids, blk_pad,
-                       ngrid, stage);
+void plan_batch_ls(std::vector<LsBatchGrid>& grids, std::vector<int> blk_start[3]) {
+  auto padded_of = [](const LsBatchGrid& G) { return padded(Dims{G.nx, G.ny, G.nz}); };
+  int kz = 16;
+  long long n;
+  do {
+    kz /= 2;
+    n = 0;
+    for (const LsBatchGrid& G : grids) {
+      const PDims g = padded_of(G);
+      n += adv_blocks(g, 2, adv_ltx(g), kz);
+    }
+  } while (kz > 2 && n < 1024);
+  for (int s = 0; s < 3; s++) {
+    blk_start[s].assign(1, 0);
+    for (LsBatchGrid& G : grids) {
+      const PDims g = padded_of(G);
+      G.ltx = adv_ltx(g);
+      G.kz = kz;
+      blk_start[s].push_back(blk_start[s].back() + adv_blocks(g, s, G.ltx, kz));
+    }
+  }
+}
+
+int op_batch_ls_step(hipStream_t st, const LsBatchGrid* grids, int* const blk_start[3],
+                     const int nblk[3], int ngrid) {
+  hipLaunchKernelGGL(k_batch_advect<0>, dim3(nblk[0]), dim3(256), 0, st, grids, blk_start[0], ngrid);
+  hipLaunchKernelGGL(k_batch_advect<1>, dim3(nblk[1]), dim3(256), 0, st, grids, blk_start[1], ngrid);
+  hipLaunchKernelGGL(k_batch_advect<2>, dim3(nblk[2]), dim3(256), 0, st, grids, blk_start[2], ngrid);
   EMX_TRY_HIP(hipGetLastError());
   return EMX_OK;
 }
@@ -854,44 +909,26 @@ int op_ls_reinit(emx_ctx* ctx, double* phi, const double* jbn, const double* dmi
   const long long N = d.N(), NG = g.N();
   double* P = ctx->ls_buf;  // the iteration's phi, ping-pong with Q
   double* Q = P + NG;
-  double* J1 = Q + NG;
-  double* J5 = J1 + NG;
-  double* J9 = J5 + NG;
-  double* Dm = J9 + NG;
-  double* T1 = Dm + NG;
+  double* T1 = Q + NG;
   double* T2 = T1 + NG;
   hipStream_t st = ctx->stream;
-  const unsigned bg = blocks_for(NG);
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-            hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, phi, d.nx, d.ny, d.nz, P, g));
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-            hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, dmin, d.nx, d.ny, d.nz, Dm, g));
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-            hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, jbn, d.nx, d.ny, d.nz, J1, g));
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-            hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, jbn + 4 * N, d.nx, d.ny, d.nz,
-                               J5, g));
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-            hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, jbn + 8 * N, d.nx, d.ny, d.nz,
-                               J9, g));
-  // Dev1thO_Downwind receives 1.0/deltaX (lsTransportEc.cu:487-495)
+  EMX_TIMED(ctx, "ls_pad", 8.0 * (N + NG),
+            hipLaunchKernelGGL(k_pad, dim3(blocks_for(NG)), dim3(256), 0, st, phi, d.nx, d.ny,
+                               d.nz, P, g));
   const double iX = 1.0 / dx, iY = 1.0 / dy, iZ = 1.0 / dz, dt = 0.5 * deltamin;
   // the padding already mirrors the ghost layers of the first iteration
   for (int it = 1; it <= 10; it++) {
-    // per point: src, three metrics, phi (= phi0), dmin, out
-    EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              launch_reinit_stage<0>(st, P, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, T1));
-    EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              launch_reinit_stage<1>(st, T1, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, T2));
-    EMX_TIMED(ctx, "ls_reinit_stage", 56.0 * NG,
-              launch_reinit_stage<2>(st, T2, P, Dm, J1, J5, J9, g, iX, iY, iZ, dt, Q));
-    double* t = P;
-    P = Q;
-    Q = t;
+    // per point: src, phi (= phi0), out; three metrics and dmin, interior
+    // fields.  The last iteration writes phi itself.
+    EMX_TIMED(ctx, "ls_reinit_stage", 16.0 * NG + 32.0 * N,
+              launch_reinit_stage<0>(st, P, P, dmin, jbn, g, iX, iY, iZ, dt, T1));
+    EMX_TIMED(ctx, "ls_reinit_stage", 24.0 * NG + 32.0 * N,
+              launch_reinit_stage<1>(st, T1, P, dmin, jbn, g, iX, iY, iZ, dt, T2));
+    EMX_TIMED(ctx, "ls_reinit_stage", 24.0 * NG + 32.0 * N,
+              launch_reinit_stage<2>(st, T2, P, dmin, jbn, g, iX, iY, iZ, dt, Q,
+                                     it == 10 ? phi : nullptr));
+    std::swap(P, Q);
   }
-  EMX_TIMED(ctx, "ls_unpad", 16.0 * N,
-            hipLaunchKernelGGL(k_unpad, dim3(blocks_for(N)), dim3(256), 0, st, P, g, d.nx, d.ny,
-                               d.nz, phi));
   EMX_TRY_HIP(hipGetLastError());
   return EMX_OK;
 }
@@ -902,25 +939,21 @@ int op_ls_advect_weno5(emx_ctx* ctx, double* phi, const double* vel,
   const Dims d = ctx->d;
   const PDims g = padded(d);
   const long long N = d.N(), NG = g.N();
-  double* P = ctx->ls_buf;
-  double* T1 = P + NG;
+  double* T1 = ctx->ls_buf;
   double* T2 = T1 + NG;
-  hipStream_t st = ctx->stream;
-  const unsigned bg = blocks_for(NG);
-  EMX_TIMED(ctx, "ls_pad", 16.0 * NG,
-          hipLaunchKernelGGL(k_pad, dim3(bg), dim3(256), 0, st, phi, d.nx, d.ny, d.nz, P, g));
   const double iX = 1.0 / dx, iY = 1.0 / dy, iZ = 1.0 / dz;
-  // per stage: phi in (and the step's phi) and phi out on the padded grid;
-  // the velocity and the metrics once on the interior grid
-  EMX_TIMED(ctx, "ls_weno_stage", 16.0 * NG + 48.0 * N,
-          hipLaunchKernelGGL(k_weno_stage, dim3(bg), dim3(256), 0, st, 0, P, P, vel, jbn, g,
-                     iX, iY, iZ, dt, T1, nullptr));
-  EMX_TIMED(ctx, "ls_weno_stage", 24.0 * NG + 48.0 * N,
-          hipLaunchKernelGGL(k_weno_stage, dim3(bg), dim3(256), 0, st, 1, T1, P, vel, jbn, g,
-                     iX, iY, iZ, dt, T2, nullptr));
-  EMX_TIMED(ctx, "ls_weno_stage", 16.0 * NG + 56.0 * N,
-          hipLaunchKernelGGL(k_weno_stage, dim3(bg), dim3(256), 0, st, 2, T2, P, vel, jbn, g,
-                     iX, iY, iZ, dt, nullptr, phi));
+  const int ltx = adv_ltx(g);
+  int kz = 8;
+  while (kz > 2 && adv_blocks(g, 2, ltx, kz) < 1024) kz /= 2;
+  auto go = [&](auto kern, int stage, const double* src, double* out) {
+    hipLaunchKernelGGL(kern, dim3(adv_blocks(g, stage, ltx, kz)), dim3(256), 0, ctx->stream, src,
+                       phi, vel, jbn, g, ltx, kz, iX, iY, iZ, dt, out);
+  };
+  // per stage: the stage's phi in and out, the step's phi, the velocity and
+  // the metrics
+  EMX_TIMED(ctx, "ls_weno_stage", 8.0 * NG + 56.0 * N, go(k_ls_advect<0>, 0, phi, T1));
+  EMX_TIMED(ctx, "ls_weno_stage", 16.0 * NG + 56.0 * N, go(k_ls_advect<1>, 1, T1, T2));
+  EMX_TIMED(ctx, "ls_weno_stage", 8.0 * NG + 64.0 * N, go(k_ls_advect<2>, 2, T2, phi));
   EMX_TRY_HIP(hipGetLastError());
   return EMX_OK;
 }

@@ -86,16 +86,17 @@ struct LsBatchGrid {
   double* phi;
   const double* vel;
   const double* jbn;  // the box's metrics (11 components, interior grid)
-  double* P;
-  double* T1;
+  double* T1;         // padded stage results
   double* T2;
   double iX, iY, iZ, dt;
+  int ltx, kz;  // tile shape, set by plan_batch_ls
 };
 long long ls_padded_points(int nx, int ny, int nz);
-// blk_pad: per-grid first workgroup (ngrid + 1 entries) over the padded
-// points, 256 points per workgroup.
-int op_batch_ls_step(hipStream_t st, const LsBatchGrid* grids, const int* blk_pad,
-                     int nblk_pad, int ngrid);
+// Sets the tile shapes; blk_start[s]: per-grid first workgroup (ngrid + 1
+// entries) of stage s.
+void plan_batch_ls(std::vector<LsBatchGrid>& grids, std::vector<int> blk_start[3]);
+int op_batch_ls_step(hipStream_t st, const LsBatchGrid* grids, int* const blk_start[3],
+                     const int nblk[3], int ngrid);
 
 // level set (levelset.hip); scratch is ctx->ls_buf
 size_t ls_scratch_doubles(const Dims& d);
