@@ -226,7 +226,11 @@ int op_sgdm(emx_ctx* ctx, const double* u, const double* dvel,
 // filter of ratio 2, weights (1/4, 1/2, 1/4) per direction with clamped
 // indices at the walls, applied along x, then y, then z.
 //
-// Two kernels, both on the plane march of k_sgs_fused: a workgroup owns a
+// Two kernels:
+//   k_dynsmag_lm:  the 21 quantities S (6), |S| S (6), u_a u_b (6), u (3)
+//                  -> L:M and M:M (two fields of scratch), delta^2 |S|;
+//   k_dynsmag_nut: the filtered L:M and M:M -> C, nu_t, vis.
+// The second is on the plane march of k_sgs_fused: a workgroup owns a
 // 32 x 8 (i, j) tile and a slab of k planes.  For each plane (and one
 // clamped plane either side of the slab) it forms the filtered quantities
 // at the tile and its one-point halo into LDS, filters them along x and y
@@ -234,22 +238,18 @@ int op_sgdm(emx_ctx* ctx, const double* u, const double* dvel,
 //   Z(k) = (1/4 Y(k-1) + 1/2 Y(k)) + 1/4 Y(k+1),
 // the term of plane k+1 added when that plane arrives, so every quantity
 // of a point is formed once per plane and read once from memory.
-//   k_dynsmag_lm:  the 21 quantities S (6), |S| S (6), u_a u_b (6), u (3)
-//                  -> L:M and M:M (two fields of scratch);
-//   k_dynsmag_nut: the filtered L:M and M:M -> C, nu_t, vis.
 constexpr int DS_TX = 32, DS_TY = 8, DS_HX = DS_TX + 2, DS_HY = DS_TY + 2,
-              DS_HP = DS_HX * DS_HY, DS_KS = 16;
+              DS_HP = DS_HX * DS_HY;
 
 // Strain-rate pairs (0,0) (1,1) (2,2) (0,1) (0,2) (1,2); off-diagonal pairs
 // count twice in contractions.
-__device__ __forceinline__ void strain(const double* dvel, const double* jbn, long long N,
-                                       long long q, double S[6], double* aS) {
-  const double m[3] = {jbn[q], jbn[4 * N + q], jbn[8 * N + q]};
+__device__ __forceinline__ void strain(const double m[3], const double dv[9], double S[6],
+                                       double* aS) {
   double g[9];
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
-    for (int b = 0; b < 3; b++) g[3 * a + b] = m[b] * dvel[(3 * b + a) * N + q];
+    for (int b = 0; b < 3; b++) g[3 * a + b] = m[b] * dv[3 * b + a];
   const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
   double s2 = 0.0;
 #pragma unroll
@@ -260,20 +260,31 @@ __device__ __forceinline__ void strain(const double* dvel, const double* jbn, lo
   *aS = sqrt(2.0 * s2);
 }
 
-// The plane march shared by both kernels.  form(q, v) writes the NQ
+// |S| at point q.
+__device__ __forceinline__ double strain_norm(const double* dvel, const double* jbn, long long N,
+                                              long long q) {
+  const double m[3] = {jbn[q], jbn[4 * N + q], jbn[8 * N + q]};
+  double dv[9], S[6], aS;
+#pragma unroll
+  for (int k = 0; k < 9; k++) dv[k] = dvel[k * N + q];
+  strain(m, dv, S, &aS);
+  return aS;
+}
+
+// The plane march of k_dynsmag_nut.  form(q, v) writes the NQ
 // quantities of grid point q; done(p, Z) receives the filtered quantities
 // of an owned point p of the slab.  Planes k0-1 .. k1 are formed (clamped
 // into the grid); when plane kk arrives, Z(kk-1) is completed and handed
 // to done(), Z(kk) gets its middle term and Z(kk+1) its first.
 template <int NQ, class Form, class Done>
-__device__ __forceinline__ void dyn_march(const Dims& d, double (*Q)[DS_HP], Form form,
+__device__ __forceinline__ void dyn_march(const Dims& d, int kz, double (*Q)[DS_HP], Form form,
                                           Done done) {
   const long long sy = d.nx, sz = (long long)d.nx * d.ny;
   const int tx = threadIdx.x % DS_TX, ty = threadIdx.x / DS_TX;
   const unsigned nbx = (d.nx + DS_TX - 1) / DS_TX, nby = (d.ny + DS_TY - 1) / DS_TY;
   const unsigned b = xcd_block(blockIdx.x, gridDim.x);
   const int i0 = (int)(b % nbx) * DS_TX, j0 = (int)((b / nbx) % nby) * DS_TY;
-  const int k0 = (int)(b / (nbx * nby)) * DS_KS, k1 = min(k0 + DS_KS, d.nz);
+  const int k0 = (int)(b / (nbx * nby)) * kz, k1 = min(k0 + kz, d.nz);
   const int i = i0 + tx, j = j0 + ty;
   const bool own = i < d.nx && j < d.ny;
   const int hc = (ty + 1) * DS_HX + (tx + 1);
@@ -314,92 +325,193 @@ __device__ __forceinline__ void dyn_march(const Dims& d, double (*Q)[DS_HP], For
 // L:M and M:M at each point: with hat() the test filter,
 //   L_ij = hat(u_i u_j) - hat(u_i) hat(u_j),
 //   M_ij = 2 delta^2 (hat(|S| S_ij) - 4 |hat S| hat S_ij).
-__global__ void __launch_bounds__(256)
+// Where dS is given it takes delta^2 |S|.
+//
+// A workgroup of 512 owns 30 x 14 columns; its work-items hold these and one
+// more on every side (clamped indices), 32 columns to a row, and march z
+// through a slab of kz planes with the next plane's 16 inputs in flight.
+// Per plane a work-item forms its 21 quantities, filters them along y from
+// its neighbours' rows in LDS, along x by lane shifts and along z in
+// registers, all with the weights (1, 2, 1); the common factor 1/64 is a
+// power of two.  Bound by issue and LDS when 256 work-items formed the 340
+// points of a 32 x 8 tile and its halo in two rounds and each read the nine
+// points of every quantity's plane stencil (885 vector and 240 LDS
+// operations per point-wave): 500 us at 224 x 192 x 160, 358 us now (2.9 TB/s,
+// two wavefronts per SIMD); k_dynsmag_nut 202 us when it formed |S| again from
+// dvel, 72 us with delta^2 |S| stored.
+constexpr int DL_W = 32, DL_R = 16, DL_OX = DL_W - 2, DL_OY = DL_R - 2, DL_T = DL_W * DL_R;
+
+// v of the lane below / above (within a wavefront; DPP wave shifts).
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
+
+__global__ void __launch_bounds__(DL_T)
 k_dynsmag_lm(const double* u, const double* dvel, const double* jbn, const double* delta,
-             Dims d, double* LM, double* MM) {
-  __shared__ double Q[21][DS_HP];
-  const long long N = d.N();
+             Dims d, int kz, double* LM, double* MM, double* dS) {
+  extern __shared__ double Q[];  // [21][DL_T]
+  constexpr int NQ = 21;
+  const long long N = d.N(), sz = (long long)d.nx * d.ny;
   const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
-  dyn_march<21>(
-      d, Q,
-      [&](long long q, double* v) {
-        double S[6], aS;
-        strain(dvel, jbn, N, q, S, &aS);
-        const double uq[3] = {u[q], u[N + q], u[2 * N + q]};
+  const int tid = threadIdx.x, tx = tid % DL_W, ty = tid / DL_W;
+  const unsigned nbx = (d.nx + DL_OX - 1) / DL_OX, nby = (d.ny + DL_OY - 1) / DL_OY;
+  const unsigned b = xcd_block(blockIdx.x, gridDim.x);
+  const int i = (int)(b % nbx) * DL_OX - 1 + tx, j = (int)((b / nbx) % nby) * DL_OY - 1 + ty;
+  const int k0 = (int)(b / (nbx * nby)) * kz, k1 = min(k0 + kz, d.nz);
+  const bool own = tx > 0 && tx < DL_W - 1 && ty > 0 && ty < DL_R - 1 && i < d.nx && j < d.ny;
+  const long long col = min(max(i, 0), d.nx - 1) + (long long)min(max(j, 0), d.ny - 1) * d.nx;
+  // the rows on either side (the outer rows' own: they are not owned)
+  const int up = ty > 0 ? tid - DL_W : tid, dn = ty < DL_R - 1 ? tid + DL_W : tid;
+
+  double m[3], dv[9], uq[3], dl;  // the next plane's inputs
+  auto load = [&](int k) {
+    const long long q = col + (long long)min(max(k, 0), d.nz - 1) * sz;
 #pragma unroll
-        for (int t = 0; t < 6; t++) {
-          v[t] = S[t];
-          v[6 + t] = aS * S[t];
-          v[12 + t] = uq[ia[t]] * uq[ib[t]];
-        }
+    for (int c = 0; c < 3; c++) {
+      m[c] = jbn[4 * c * N + q];
+      uq[c] = u[c * N + q];
+    }
 #pragma unroll
-        for (int c = 0; c < 3; c++) v[18 + c] = uq[c];
-      },
-      [&](long long p, const double* Z) {
-        double s2 = 0.0;
+    for (int c = 0; c < 9; c++) dv[c] = dvel[c * N + q];
+    dl = delta[q];
+  };
+  load(k0 - 1);
+  double Zn[NQ] = {}, Zc[NQ] = {};  // Z(kk+1) after its first term, Z(kk) after two
+  double d2p = 0.0;                 // delta^2 of plane kk-1
+  for (int kk = k0 - 1; kk <= k1; kk++) {
+    double v[NQ];
+    double aS;
+    strain(m, dv, v, &aS);
 #pragma unroll
-        for (int t = 0; t < 6; t++) s2 += (t < 3 ? 1.0 : 2.0) * Z[t] * Z[t];
-        const double ahS = sqrt(2.0 * s2);
-        const double d2 = delta[p] * delta[p];
-        double lm = 0.0, mm = 0.0;
+    for (int t = 0; t < 6; t++) {
+      v[6 + t] = aS * v[t];
+      v[12 + t] = uq[ia[t]] * uq[ib[t]];
+    }
 #pragma unroll
-        for (int t = 0; t < 6; t++) {
-          const double L = Z[12 + t] - Z[18 + ia[t]] * Z[18 + ib[t]];
-          const double M = 2.0 * d2 * (Z[6 + t] - 4.0 * ahS * Z[t]);
-          const double wq = t < 3 ? 1.0 : 2.0;
-          lm += wq * L * M;
-          mm += wq * M * M;
-        }
-        LM[p] = lm;
-        MM[p] = mm;
-      });
+    for (int c = 0; c < 3; c++) v[18 + c] = uq[c];
+    const double d2 = dl * dl;
+    if (kk < k1) load(kk + 1);
+#pragma unroll
+    for (int t = 0; t < NQ; t++) Q[t * DL_T + tid] = v[t];
+    if (dS && own && kk >= k0 && kk < k1) dS[col + kk * sz] = d2 * aS;
+    lds_barrier();
+    double Zd[NQ];
+#pragma unroll
+    for (int t = 0; t < NQ; t++) {
+      const double Y = __builtin_fma(2.0, v[t], Q[t * DL_T + up] + Q[t * DL_T + dn]);
+      const double X = __builtin_fma(2.0, Y, lane_shift<DPP_WAVE_SHR1>(Y) +
+                                                 lane_shift<DPP_WAVE_SHL1>(Y));
+      Zd[t] = Zc[t] + X;                       // Z(kk-1), valid for kk > k0
+      Zc[t] = __builtin_fma(2.0, X, Zn[t]);    // Z(kk), valid for kk >= k0
+      Zn[t] = X;                               // Z(kk+1)
+    }
+    if (own && kk > k0) {
+#pragma unroll
+      for (int t = 0; t < NQ; t++) Zd[t] *= 1.0 / 64.0;
+      double s2 = 0.0;
+#pragma unroll
+      for (int t = 0; t < 6; t++) s2 += (t < 3 ? 1.0 : 2.0) * Zd[t] * Zd[t];
+      const double ahS = sqrt(2.0 * s2);
+      double lm = 0.0, mm = 0.0;
+#pragma unroll
+      for (int t = 0; t < 6; t++) {
+        const double L = Zd[12 + t] - Zd[18 + ia[t]] * Zd[18 + ib[t]];
+        const double M = 2.0 * d2p * (Zd[6 + t] - 4.0 * ahS * Zd[t]);
+        const double wq = t < 3 ? 1.0 : 2.0;
+        lm += wq * L * M;
+        mm += wq * M * M;
+      }
+      const long long p = col + (long long)(kk - 1) * sz;
+      LM[p] = lm;
+      MM[p] = mm;
+    }
+    d2p = d2;
+    lds_barrier();  // Q is rewritten for the next plane
+  }
 }
 
 // nu_t = max(0, C delta^2 |S|) with C = hat(L:M) / hat(M:M) (0 where
-// hat(M:M) <= 0); vis = c4 + nu_t when vis is not NULL.
+// hat(M:M) <= 0); vis = c4 + nu_t when vis is not NULL.  STORED: nut holds
+// delta^2 |S|, which k_dynsmag_lm left there (5 fields to move instead of 17).
+template <bool STORED>
 __global__ void __launch_bounds__(256)
 k_dynsmag_nut(const double* LM, const double* MM, const double* dvel, const double* jbn,
-              const double* delta, Dims d, double* nut, double c4, double* vis) {
+              const double* delta, Dims d, int kz, double* nut, double c4, double* vis) {
   __shared__ double Q[2][DS_HP];
   const long long N = d.N();
   dyn_march<2>(
-      d, Q,
+      d, kz, Q,
       [&](long long q, double* v) {
         v[0] = LM[q];
         v[1] = MM[q];
       },
       [&](long long p, const double* Z) {
-        double S[6], aS;
-        strain(dvel, jbn, N, p, S, &aS);
         const double C = Z[1] > 0.0 ? Z[0] / Z[1] : 0.0;
-        const double v = C * delta[p] * delta[p] * aS;
+        const double v = C * (STORED ? nut[p] : delta[p] * delta[p] * strain_norm(dvel, jbn, N, p));
         const double nu = v > 0.0 ? v : 0.0;
         nut[p] = nu;
         if (vis) vis[p] = c4 * 1.0 + nu;  // viscosidad (solver/viscosidad_incomp.f90:15-17)
       });
 }
 
-// Launches the two kernels; LM and MM are 2*N doubles of scratch.
+// Planes per slab of k_dynsmag_lm: one workgroup to a compute unit (its LDS
+// and registers), each round of 256 workgroups taking kz + 2 planes; the kz
+// with the fewest planes in all.
+static int dynsmag_slab(long long columns, int nz) {
+  int best = nz;
+  long long least = -1;
+  for (int slabs = 1; slabs <= nz; slabs++) {
+    const int kz = (nz + slabs - 1) / slabs;
+    const long long cost = (columns * ((nz + kz - 1) / kz) + 255) / 256 * (kz + 2);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = kz;
+    }
+  }
+  return best;
+}
+
+// Launches the two kernels; LM and MM are 2*N doubles of scratch.  nut is
+// also the place of delta^2 |S| between them, unless it overlaps an input
+// (the first kernel reads those at its neighbours' points).
 int launch_dynsmag(emx_ctx* ctx, hipStream_t stream, const Dims& d, const double* u,
                    const double* dvel, const double* jbn, const double* delta, double* nut,
                    double c4, double* vis, double* LM, double* MM) {
   const long long N = d.N();
-  const unsigned tiles = (unsigned)((d.nx + DS_TX - 1) / DS_TX) *
-                         (unsigned)((d.ny + DS_TY - 1) / DS_TY) *
-                         (unsigned)((d.nz + DS_KS - 1) / DS_KS);
-  // reads u(3), dvel(9), jbn(3), delta; writes LM, MM / reads LM, MM,
-  // dvel(9), jbn(3), delta; writes nut (and vis)
+  // slabs of 16 planes for k_dynsmag_nut, fewer while the chip's 256 compute
+  // units would get less than four workgroups
+  const long long tiles = (long long)((d.nx + DS_TX - 1) / DS_TX) * ((d.ny + DS_TY - 1) / DS_TY);
+  int nut_kz = 16;
+  while (nut_kz > 2 && tiles * ((d.nz + nut_kz - 1) / nut_kz) < 1024) nut_kz /= 2;
+  const unsigned nut_blocks = (unsigned)(tiles * ((d.nz + nut_kz - 1) / nut_kz));
+  const long long columns =
+      (long long)((d.nx + DL_OX - 1) / DL_OX) * ((d.ny + DL_OY - 1) / DL_OY);
+  const int kz = dynsmag_slab(columns, d.nz);
+  const unsigned lm_blocks = (unsigned)(columns * ((d.nz + kz - 1) / kz));
+  auto apart = [&](const double* f, long long n) { return nut + N <= f || f + n <= nut; };
+  const bool stored = apart(u, 3 * N) && apart(dvel, 9 * N) && apart(jbn, 11 * N) &&
+                      apart(delta, N);
+  const size_t lds = (size_t)21 * DL_T * sizeof(double);
+  EMX_TRY_HIP(hipFuncSetAttribute((const void*)k_dynsmag_lm,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // reads u(3), dvel(9), jbn(3), delta; writes LM, MM (and delta^2 |S|) /
+  // reads LM, MM and delta^2 |S|; writes nut (and vis)
   auto lm = [&] {
-    hipLaunchKernelGGL(k_dynsmag_lm, dim3(tiles), dim3(256), 0, stream, u, dvel, jbn, delta, d,
-                       LM, MM);
+    hipLaunchKernelGGL(k_dynsmag_lm, dim3(lm_blocks), dim3(DL_T), lds, stream, u, dvel, jbn,
+                       delta, d, kz, LM, MM, stored ? nut : nullptr);
   };
   auto nu = [&] {
-    hipLaunchKernelGGL(k_dynsmag_nut, dim3(tiles), dim3(256), 0, stream, LM, MM, dvel, jbn,
-                       delta, d, nut, c4, vis);
+    hipLaunchKernelGGL(stored ? k_dynsmag_nut<true> : k_dynsmag_nut<false>, dim3(nut_blocks),
+                       dim3(256), 0, stream, LM, MM, dvel, jbn, delta, d, nut_kz, nut, c4, vis);
   };
   if (ctx) {
-    EMX_TIMED(ctx, "dynsmag_lm", 18.0 * 8.0 * N, lm());
-    EMX_TIMED(ctx, "dynsmag_nut", (vis ? 17.0 : 16.0) * 8.0 * N, nu());
+    EMX_TIMED(ctx, "dynsmag_lm", (stored ? 19.0 : 18.0) * 8.0 * N, lm());
+    EMX_TIMED(ctx, "dynsmag_nut", ((stored ? 4.0 : 16.0) + (vis ? 1.0 : 0.0)) * 8.0 * N, nu());
   } else {
     lm();
     nu();
