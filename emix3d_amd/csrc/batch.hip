@@ -60,6 +60,7 @@ static void* batched_wave_kernel(int C) {
   switch (C) {
     case 1: return (void*)k_lines_batched_wave<S, 1, ProbGradDiv>;
     case 2: return (void*)k_lines_batched_wave<S, 2, ProbGradDiv>;
+    case 3: return (void*)k_lines_batched_wave<S, 3, ProbGradDiv>;
     case 4: return (void*)k_lines_batched_wave<S, 4, ProbGradDiv>;
     default: return (void*)k_lines_batched_wave<S, 8, ProbGradDiv>;
   }
@@ -117,6 +118,7 @@ struct emx_batch {
   emx::BatchLines<emx::ProbGradDiv>* lines_d[3] = {nullptr, nullptr, nullptr};
   std::vector<emx::BatchWaveLines<emx::ProbGradDiv>> waves_h;  // direction 0
   emx::BatchWaveLines<emx::ProbGradDiv>* waves_d = nullptr;
+  int wave_C = 1;  // longest chunk of a box in waves_h
   int* blk_d[3] = {nullptr, nullptr, nullptr};
   int nblk[3] = {0, 0, 0};
   int threads[3] = {0, 0, 0};
@@ -185,11 +187,13 @@ bool shape_fits(const emx_batch* b, int dir, BatchShape s) {
 }
 
 // Direction 0 on the wavefront kind: kWaveLinesPerBlock lines per workgroup,
-// each box with its shortest chunk (LDS sized for the longest, s.C).
+// each box with its shortest chunk.  The kernel and its LDS are those of the
+// longest chunk in use (three points take 93 registers, four 108).
 int plan_wave_lines(emx_batch* b, BatchShape s) {
   auto& H = b->waves_h;
   H.assign(b->nbox, BatchWaveLines<ProbGradDiv>{});
   std::vector<int> blk(b->nbox + 1, 0);
+  int longest = 1;
   for (int i = 0; i < b->nbox; i++) {
     const Dims& d = b->dims[i];
     const DirGeom g = dir_geom(d, 0);
@@ -197,6 +201,7 @@ int plan_wave_lines(emx_batch* b, BatchShape s) {
     // the shortest chunk of 1, 2, 3, 4, 8 (at most s.C) whose 64 lanes hold the line
     int C = 1;
     while (C < s.C && g.n > 64 * C) C = C == 2 ? 3 : (C == 3 ? 4 : 2 * C);
+    longest = std::max(longest, C);
     EMX_TRY(get_line_tab(b->scheme, g.n, C, KIND_WAVE, &L.T));
     L.nlines = g.nlines;
     L.nyl = g.nyl;
@@ -210,10 +215,11 @@ int plan_wave_lines(emx_batch* b, BatchShape s) {
     blk[i + 1] = blk[i] + L.nblk;
   }
   b->shape[0] = s;
+  b->wave_C = longest;
   b->nblk[0] = blk[b->nbox];
   b->threads[0] = 256;
-  b->lds[0] = wave_lds(s.C);
-  void* k = batched_kernel_for(b->scheme, 0, s.C, 256);
+  b->lds[0] = wave_lds(longest);
+  void* k = batched_kernel_for(b->scheme, 0, longest, 256);
   if (b->lds[0] > 65536)
     EMX_TRY_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)b->lds[0]));
@@ -272,7 +278,8 @@ int plan_lines(emx_batch* b, int dir, BatchShape s) {
 }
 
 int launch_pass(emx_batch* b, int dir) {
-  void* k = batched_kernel_for(b->scheme, b->shape[dir].lg, b->shape[dir].C,
+  const int lg = b->shape[dir].lg;
+  void* k = batched_kernel_for(b->scheme, lg, lg == 0 ? b->wave_C : b->shape[dir].C,
                                b->threads[dir]);
   const void* grids = b->shape[dir].lg == 0 ? (const void*)b->waves_d : (const void*)b->lines_d[dir];
   const int* blk = b->blk_d[dir];

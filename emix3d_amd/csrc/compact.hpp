@@ -203,6 +203,7 @@ __device__ __forceinline__ int line_group(int bxp, int gx) {
 // LDS in the lanes' chunk order (see lines_wave_body).
 struct WaveTabs {
   const double *ib, *m, *gam1, *H, *G, *af, *ab;
+  int ks;  // LineTab::KS
 };
 
 // Stages the wavefront kind's tables into lds (5*64*C + 768 doubles) in the
@@ -283,9 +284,12 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
+        if (k >= wt.ks) continue;
         double up[F];
 #pragma unroll
-        for (int f = 0; f < F; f++) up[f] = __shfl_up(B[f], d, 64);
+        for (int f = 0; f < F; f++)
+          up[f] = k == 0 ? lane_below(B[f])
+                         : (k == 1 ? lane_below(lane_below(B[f])) : __shfl_up(B[f], d, 64));
         if (lane >= d) {
 #pragma unroll
           for (int f = 0; f < F; f++) B[f] += wt.af[k * 64 + lane] * up[f];
@@ -293,8 +297,7 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
       }
 #pragma unroll
       for (int f = 0; f < F; f++) {
-        double Y = __shfl_up(B[f], 1, 64);
-        if (lane == 0) Y = 0.0;
+        const double Y = lane_below(B[f]);
 #pragma unroll
         for (int q = 0; q < C; q++) {
           const int l = s + q;
@@ -325,9 +328,12 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
+        if (k >= wt.ks) continue;
         double dn[F];
 #pragma unroll
-        for (int f = 0; f < F; f++) dn[f] = __shfl_down(B[f], d, 64);
+        for (int f = 0; f < F; f++)
+          dn[f] = k == 0 ? lane_above(B[f])
+                         : (k == 1 ? lane_above(lane_above(B[f])) : __shfl_down(B[f], d, 64));
         if (lane + d < 64) {
 #pragma unroll
           for (int f = 0; f < F; f++) B[f] += wt.ab[k * 64 + lane] * dn[f];
@@ -335,8 +341,7 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
       }
 #pragma unroll
       for (int f = 0; f < F; f++) {
-        double X = __shfl_down(B[f], 1, 64);
-        if (lane == 63) X = 0.0;
+        const double X = lane_above(B[f]);
 #pragma unroll
         for (int q = 0; q < C; q++) {
           const int l = s + q;
@@ -400,7 +405,7 @@ __device__ __forceinline__ void lines_wave_body(const Prob& prob, const LineTab&
   double* s_G = s_H + TS;
   double* s_af = s_G + TS;    // Af[384] Ab[384]
   double* s_ab = s_af + 384;
-  const WaveTabs wt{s_ib, s_m, s_gam1, s_H, s_G, s_af, s_ab};
+  const WaveTabs wt{s_ib, s_m, s_gam1, s_H, s_G, s_af, s_ab, T.KS};
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   double* xb = s_ab + 384 + wv * 64 * STR;
   const long long stride = (long long)nblk * 4;
@@ -759,8 +764,8 @@ k_lines_batched_wave(const BatchWaveLines<Prob>* grids, const int* blk_start, in
   else if (CMAX >= 4 && G.T.C == 4)
     lines_wave_body<S, (CMAX >= 4 ? 4 : 1)>(prob, G.T, G.nlines, G.nyl, G.sj, G.sk, G.sl,
                                              G.ih, blk, G.nblk);
-  else if (CMAX >= 4 && G.T.C == 3)
-    lines_wave_body<S, (CMAX >= 4 ? 3 : 1)>(prob, G.T, G.nlines, G.nyl, G.sj, G.sk, G.sl,
+  else if (CMAX >= 3 && G.T.C == 3)
+    lines_wave_body<S, (CMAX >= 3 ? 3 : 1)>(prob, G.T, G.nlines, G.nyl, G.sj, G.sk, G.sl,
                                              G.ih, blk, G.nblk);
   else if (CMAX >= 2 && G.T.C == 2)
     lines_wave_body<S, (CMAX >= 2 ? 2 : 1)>(prob, G.T, G.nlines, G.nyl, G.sj, G.sk, G.sl,

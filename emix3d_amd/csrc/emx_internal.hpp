@@ -66,6 +66,18 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// v of the wavefront's next lower / higher lane (0 at the end), by DPP wave
+// shifts: vector instructions, where a shuffle takes two of LDS.
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_below(double v) { return dpp_shift<0x138>(v); }
+__device__ __forceinline__ double lane_above(double v) { return dpp_shift<0x130>(v); }
+
 // Kinds of line solver launch (see compact.hpp).
 enum LineKind {
   KIND_WAVE = 0,       // one wavefront per line, lanes along the line
@@ -96,6 +108,7 @@ struct LineTab {
   int kind;   // LineKind
   int K;      // chunk carries further than K chunks away are below 1e-24
   int KB;     // max(K, 1): width of the banded carry weights
+  int KS;     // wave-scan steps; the multipliers of later ones are below 1e-24
   // all arrays below live in one device block (blob), laid out as
   //   ib[n] m[n] gam[n+1] H[n] G[n] | Af[384] Ab[384] | WfB[P*KB] WbB[P*KB]
   //   | Wf[P*P] Wb[P*P]

@@ -181,6 +181,9 @@ int build_tab(int scheme_flags, int n, int C, int kind, LineTab* t, double cfilt
       }
     }
   }
+  int KS = 0;
+  for (int t = 0; t < 6 * 64; t++)
+    if (std::max(std::fabs(Af[t]), std::fabs(Ab[t])) >= 1e-24) KS = t / 64 + 1;
   // banded carry weights of the strided kinds: WfB[c*KB+k] = Wf[c][c-1-k],
   // WbB[c*KB+k] = Wb[c][c+1+k], k < KB
   const int KB = std::max(K, 1);
@@ -232,6 +235,7 @@ int build_tab(int scheme_flags, int n, int C, int kind, LineTab* t, double cfilt
   t->kind = kind;
   t->K = K;
   t->KB = KB;
+  t->KS = KS;
   t->blob = dev;
   t->ib = dev + off[0];
   t->m = dev + off[1];

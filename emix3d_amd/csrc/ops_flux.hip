@@ -110,7 +110,7 @@ k_flux_project_xi(FluxIn F, LineTab T, long long nlines, int nx, int ny, int yz,
   // uses their rows (2*TS >= 64*(C+1) doubles) as its transpose buffer once
   // it has read them: no other wave touches them before the next line.
   const WaveTabs wt{lds, lds + TS, lds + 2 * TS, lds + 3 * TS, lds + 4 * TS, lds + 5 * TS,
-                    lds + 5 * TS + 384};
+                    lds + 5 * TS + 384, T.KS};
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   double* lineF = lds + 5 * TS + 768;  // [8][TS]
   double* xb = lineF + 2 * wv * TS;

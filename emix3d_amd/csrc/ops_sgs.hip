@@ -341,16 +341,6 @@ __device__ __forceinline__ void dyn_march(const Dims& d, int kz, double (*Q)[DS_
 // dvel, 72 us with delta^2 |S| stored.
 constexpr int DL_W = 32, DL_R = 16, DL_OX = DL_W - 2, DL_OY = DL_R - 2, DL_T = DL_W * DL_R;
 
-// v of the lane below / above (within a wavefront; DPP wave shifts).
-template <int CTRL>
-__device__ __forceinline__ double lane_shift(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-constexpr int DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
-
 __global__ void __launch_bounds__(DL_T)
 k_dynsmag_lm(const double* u, const double* dvel, const double* jbn, const double* delta,
              Dims d, int kz, double* LM, double* MM, double* dS) {
@@ -404,8 +394,8 @@ k_dynsmag_lm(const double* u, const double* dvel, const double* jbn, const doubl
 #pragma unroll
     for (int t = 0; t < NQ; t++) {
       const double Y = __builtin_fma(2.0, v[t], Q[t * DL_T + up] + Q[t * DL_T + dn]);
-      const double X = __builtin_fma(2.0, Y, lane_shift<DPP_WAVE_SHR1>(Y) +
-                                                 lane_shift<DPP_WAVE_SHL1>(Y));
+      const double X = __builtin_fma(2.0, Y, lane_below(Y) +
+                                                 lane_above(Y));
       Zd[t] = Zc[t] + X;                       // Z(kk-1), valid for kk > k0
       Zc[t] = __builtin_fma(2.0, X, Zn[t]);    // Z(kk), valid for kk >= k0
       Zn[t] = X;                               // Z(kk+1)
