@@ -201,8 +201,8 @@ def main():
 # known size, 1.9998 and 1.0), keyed by the kernel label (the accumulation
 # passes: the average over their eta and zeta launches);
 # profiles/rk_stage_256_c6f_hbm_traffic.md holds the runs.
-MEASURED_TRAFFIC = {"flux_div_all[accumulate]": 881288263.0, "flux_project_xi": 6174124426.0,
-                    "sgdm": 3716755246.0}
+MEASURED_TRAFFIC = {"flux_div_all[accumulate]": 3567500000.0, "flux_project_xi": 6174124426.0,
+                    "sgdm": 3786000000.0}
 
 
 def kernel_breakdown(kernels, steps):
@@ -321,12 +321,13 @@ def glue_section(op, f, jbn, sgd, c4, work, stage_s, steps, warmup):
 
     t_r = timed(reinit, max(3, steps // 4), 1)
     NG = float(n + 10) ** 3
-    # per iteration: ghost mirror (16 B) and three stages (56 + 64 + 64 B) on
-    # the padded grid; five paddings and the unpadding; the copy of phi_init
-    r_bytes = (10 * (16 + 184) + 5 * 16) * NG + 16 * N + 16 * N
-    # FILTRADO: 15 line passes (field, J, 1/J in; field out) + the
-    # primitive variables (um1 1..5 in; u, pres, temp out)
-    f_bytes = (15 * 4 + 10) * 8.0 * N
+    # per iteration three stages (16 + 24 + 24 B on the padded grid, the
+    # metrics and deltamin, 32 B each, on the interior one); the padding of
+    # phi and the copy of phi_init
+    r_bytes = 10 * (64 * NG + 96 * N) + 8 * (N + NG) + 16 * N
+    # FILTRADO: one launch per direction (five fields, J, 1/J in; five fields
+    # out) + the primitive variables (um1 1..5 in; u, pres, temp out)
+    f_bytes = (3 * 12 + 10) * 8.0 * N
     out = {"workload": f"{n}^3 device RUNGEK sub-step 2 (operator, update, boundary values, "
                        "clip, pressure extrapolation into a central solid ball of radius 0.15, "
                        "rebuild), FILTRADO(itf=1, cfilt=0.49) and the level-set "

@@ -30,7 +30,7 @@ __device__ __forceinline__ float softplus_f(float z) {
 //
 // These passes replace one-point-per-lane loops whose 64 activations per
 // layer, indexed at run time, lived in scratch memory: at 65536 rows 342 us
-// forward and 819 us backward, against 32 and 79 us now (the rows'
+// forward and 819 us backward, against 32 and 75 us now (the rows'
 // pre-activations are 50 MB, 11 us at the copy rate; the products 24 us at
 // the FP32 matrix rate of 153 TFLOP/s).  The backward pass is bound by the
 // latency of one wavefront per SIMD.
@@ -475,7 +475,7 @@ int emx_mlp_backward_f32(const float* params, const float* norm, const float* fe
                    emx_mlp_backward_work(n));
     return EMX_ERR_SIZE;
   }
-  // one workgroup of eight wavefronts per compute unit, each wavefront at
+  // one workgroup of four wavefronts per compute unit, each wavefront at
   // least one 16-row tile; the partials fit the work area for every n
   const int tiles = (n + 15) / 16;
   const int nblk = std::min(256, (tiles + emx::MG_WAVES - 1) / emx::MG_WAVES);

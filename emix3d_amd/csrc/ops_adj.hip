@@ -145,7 +145,7 @@ struct ProbDivAdj {
 // the points they overwrite with the results of all three directions.  One
 // pass per direction that scattered at once read the primal fields three
 // times and added to its outputs in memory: 1008 B per point and 3 x 236 us
-// at 128^3, against 848 B and 102 + 97 + 148 + 141 us now (4.1 TB/s in the
+// at 128^3, against 832 B and 102 + 97 + 148 + 141 us now (4.1 TB/s in the
 // scatter passes, whose registers leave two workgroups on a CU).
 struct AdjScratch {
   double* um_bar;    // 5 fields (1 is zero)
