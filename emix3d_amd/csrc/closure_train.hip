@@ -30,10 +30,11 @@ __device__ __forceinline__ float softplus_f(float z) {
 //
 // These passes replace one-point-per-lane loops whose 64 activations per
 // layer, indexed at run time, lived in scratch memory: at 65536 rows 342 us
-// forward and 819 us backward, against 32 and 75 us now (the rows'
+// forward and 819 us backward, against 32 and 65 us now (the rows'
 // pre-activations are 50 MB, 11 us at the copy rate; the products 24 us at
 // the FP32 matrix rate of 153 TFLOP/s).  The backward pass is bound by the
-// latency of one wavefront per SIMD.
+// latency of one wavefront per SIMD (75 us before the next tile's reads were
+// in flight during a tile).
 constexpr int MLP_ACT = 3 * MLP_H + 1;
 constexpr int MLP_LDW = MLP_H + 4;  // row stride in LDS: 4 banks between rows
 typedef float f32x4u __attribute__((__vector_size__(16), __aligned__(4)));
@@ -227,55 +228,70 @@ k_mlp_grad(const float* P, const float* norm, const float* feat, const float* ac
       g3[t][i] = g2[t][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
   }
-  // tiles dealt round robin over all wavefronts
-  for (int tile = wv * gridDim.x + blockIdx.x; tile < ntile; tile += nwave) {
+  // What a lane reads of a tile; rows past the end are clamped to the last
+  // one, and their zero output derivatives clear everything they reach.
+  struct Tile {
+    f32x4 z3p[4], z2p[4];                  // pre-activations, point layout
+    float z3n[4][4], z2n[4][4], z1n[4][4]; // neuron layout
+    float z4p, dp, z4n[4], dn[4], f[4];    // output neuron, dnu, input xk
+  };
+  auto load = [&](int tile) {
+    Tile T;
+    auto row = [&](int p) { return p < n ? p : n - 1; };
+    const int rp = row(16 * tile + m);
+    const float* ap = act + (long long)rp * MLP_ACT;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      T.z3p[t] = *reinterpret_cast<const f32x4u*>(ap + 2 * MLP_H + 16 * t + 4 * g);
+      T.z2p[t] = *reinterpret_cast<const f32x4u*>(ap + MLP_H + 16 * t + 4 * g);
+    }
+    T.z4p = ap[3 * MLP_H];
+    T.dp = dnu[rp];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = row(16 * tile + 4 * g + i);
+      const float* an = act + (long long)r * MLP_ACT + m;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        T.z3n[t][i] = an[2 * MLP_H + 16 * t];
+        T.z2n[t][i] = an[MLP_H + 16 * t];
+        T.z1n[t][i] = an[16 * t];
+      }
+      T.z4n[i] = an[3 * MLP_H - m];
+      T.dn[i] = dnu[r];
+      T.f[i] = feat[(long long)r * MLP_IN + xk];
+    }
+    return T;
+  };
+  // tiles dealt round robin over all wavefronts, the next one's reads in
+  // flight while a tile is worked on
+  int tile = wv * gridDim.x + blockIdx.x;
+  Tile next;
+  if (tile < ntile) next = load(tile);
+  for (; tile < ntile; tile += nwave) {
+    const Tile T = next;
+    if (tile + nwave < ntile) next = load(tile + nwave);
     reread_lds();
     const int p0 = 16 * tile;
-    const bool pin = p0 + m < n;              // point layout: point m
-    const float* ap = act + (long long)(pin ? p0 + m : n - 1) * MLP_ACT;
-    bool nin[4];                              // neuron layout: points 4g + i
-    const float* an[4];
-    float d4n[4], xn[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int p = p0 + 4 * g + i;
-      nin[i] = p < n;
-      an[i] = act + (long long)(nin[i] ? p : n - 1) * MLP_ACT;
-    }
-    // rows past the end: zero derivatives and zero inputs
-    auto load_p = [&](int layer, int t, float z[4]) {
-      const f32x4 v = *reinterpret_cast<const f32x4u*>(ap + layer * MLP_H + 16 * t + 4 * g);
-#pragma unroll
-      for (int i = 0; i < 4; i++) z[i] = pin ? v[i] : 0.0f;
-    };
-    auto load_n = [&](int layer, int t, float z[4]) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float v = an[i][layer * MLP_H + 16 * t + m];
-        z[i] = nin[i] ? v : 0.0f;
-      }
-    };
     float z3p[4][4], z3n[4][4], z2p[4][4], z2n[4][4], z1n[4][4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-      load_p(2, t, z3p[t]);
-      load_n(2, t, z3n[t]);
-    }
-    float d4p = pin ? dnu[p0 + m] * oscale * sigmoid_f(ap[3 * MLP_H]) : 0.0f;
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        z3p[t][i] = T.z3p[t][i];
+        z2p[t][i] = T.z2p[t][i];
+        z3n[t][i] = T.z3n[t][i];
+        z2n[t][i] = T.z2n[t][i];
+        z1n[t][i] = T.z1n[t][i];
+      }
+    float d4n[4], xn[4];
+    // point layout: point m; neuron layout: points 4g + i
+    const float d4p = p0 + m < n ? T.dp * oscale * sigmoid_f(T.z4p) : 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int p = nin[i] ? p0 + 4 * g + i : n - 1;
-      d4n[i] = nin[i] ? dnu[p] * oscale * sigmoid_f(an[i][3 * MLP_H]) : 0.0f;
-      const float f = feat[(long long)p * MLP_IN + xk];
-      xn[i] = !nin[i] ? 0.0f : (m == MLP_IN ? 1.0f : (f - xshift) * xscale);
+      d4n[i] = p0 + 4 * g + i < n ? T.dn[i] * oscale * sigmoid_f(T.z4n[i]) : 0.0f;
+      xn[i] = m == MLP_IN ? 1.0f : (T.f[i] - xshift) * xscale;
     }
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      load_n(1, t, z2n[t]);
-      load_p(1, t, z2p[t]);
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++) load_n(0, t, z1n[t]);
     // layer 3: d3 in both layouts, the output neuron's sums
     float d3p[4][4], d3n[4][4];
 #pragma unroll
