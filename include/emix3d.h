@@ -276,7 +276,8 @@ int emx_adam_f32(float* params, const float* grad, float* m, float* v, int n, fl
  * exact transpose of the forward entry it names (same scheme and metric
  * projection), for gradient-based use and the learned closure's training.
  * Lines of at most 512 points in every direction (EMX_ERR_SIZE otherwise).
- * Outputs are overwritten. */
+ * Outputs are overwritten; they may hold intermediate results meanwhile, so
+ * no output may overlap an input or another output. */
 
 /* out = D^T g for D = emx_deriv along dir with inverse spacing inv_h. */
 int emx_deriv_adj(emx_ctx* ctx, int dir, const double* g, double* out,
