@@ -225,6 +225,17 @@ __device__ __forceinline__ void stage_wave_tabs(const LineTab& T, double* lds) {
   }
 }
 
+// Steps of a carry scan over the lanes' values B: those whose multipliers
+// matter, and all of them where a value is an infinity or NaN, which every
+// point of the line then takes.
+template <int F>
+__device__ __forceinline__ int scan_steps(const double (&B)[F], int ks) {
+  double s = B[0];
+#pragma unroll
+  for (int f = 1; f < F; f++) s += B[f];
+  return __any(!__builtin_isfinite(s)) ? 6 : ks;
+}
+
 // Solves NV fields of one line held by a wavefront in the coalesced order
 // (v[q][a]: point q*64 + lane of field a), in place: each field moves to
 // the chunk order through the wave's LDS buffer xb (F*64*(C+1) doubles),
@@ -281,10 +292,11 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
       double B[F];
 #pragma unroll
       for (int f = 0; f < F; f++) B[f] = act ? yp[f] : 0.0;
+      const int ks = scan_steps(B, wt.ks);
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
-        if (k >= wt.ks) continue;
+        if (k >= ks) continue;
         double up[F];
 #pragma unroll
         for (int f = 0; f < F; f++)
@@ -325,10 +337,11 @@ __device__ __forceinline__ void wave_solve(double (&v)[C][NV], const WaveTabs& w
       double B[F];
 #pragma unroll
       for (int f = 0; f < F; f++) B[f] = act ? xs[f] : 0.0;
+      const int ks = scan_steps(B, wt.ks);
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         const int d = 1 << k;
-        if (k >= wt.ks) continue;
+        if (k >= ks) continue;
         double dn[F];
 #pragma unroll
         for (int f = 0; f < F; f++)

@@ -1,13 +1,18 @@
-"""Values at and beyond the ends of the double range: the level set's
-reinitialisation where phi0^2 + dmin^2 overflows (a spacing that freezes its
-points, a level set far from any interface) against the oracle, 1e-12
-normwise relative."""
+"""Values at and beyond the ends of the double range.
+
+  * An infinity or NaN at one point of a xi line reaches every point of that
+    line's derivatives, as the line's solve couples them all, and no other
+    line, for every chunk length of the wavefront kind, alone and batched;
+  * the level set's reinitialisation where phi0^2 + dmin^2 overflows (a
+    spacing that freezes its points, a level set far from any interface)
+    against the oracle, 1e-12 normwise relative.
+"""
 import numpy as np
 import pytest
 import torch
 
 from conftest import normwise_rel
-from emix3d_amd import Operator, fields
+from emix3d_amd import Batch, Operator, fields
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +27,60 @@ def two_phase(oracle, shape):
         fields.stage_fields(*shape, 63, curvilinear=True, turbulent=False)["x"].numpy())
     d = np.sqrt(((x - 0.5) ** 2).sum(0)) - 0.3
     return oracle.jacobeano(2, x), np.ascontiguousarray(d * (1.0 + 2.0 * d)), oracle.inisgdm(x)[1]
+
+
+def assert_line_only(got, clean, line):
+    """Every value of the line (j, k) non-finite, the others as in clean."""
+    bad = ~np.isfinite(got)
+    assert bad[line].all()
+    bad[line] = False
+    assert not bad.any()
+    got, clean = got.copy(), clean.copy()
+    got[line] = clean[line] = 0.0
+    assert np.array_equal(got, clean)
+
+
+# one, two, four, eight and sixteen points to a lane; a few lines past and
+# many past what one wavefront takes at a time
+@pytest.mark.parametrize("scheme", ["c4", "c6f", "c6c"])
+@pytest.mark.parametrize("shape", [(60, 9, 8), (128, 9, 8), (140, 9, 8), (256, 70, 64),
+                                   (300, 9, 8), (700, 9, 8)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_nonfinite_xi_line(scheme, shape, value):
+    nx, ny, nz = shape
+    op = Operator(*shape, scheme)
+    rng = np.random.default_rng(nx)
+    f = rng.standard_normal((4, nz, ny, nx))
+    clean = [op.derivative(dev(f[0]), 0), *op.deriv_vel(dev(f[:3]), dev(f[3]))]
+    clean = [t.cpu().numpy() for t in clean]
+    line = (5, 7)
+    f[0][line][nx // 3] = value
+    got = op.derivative(dev(f[0]), 0).cpu().numpy()
+    assert_line_only(got, clean[0], line)
+    dvel, dtemp = (t.cpu().numpy() for t in op.deriv_vel(dev(f[:3]), dev(f[3])))
+    assert_line_only(dvel[0], clean[1][0], line)  # du/dxi
+    assert np.array_equal(dvel[1:3], clean[1][1:3])  # the fields solved beside u
+    assert np.array_equal(dtemp, clean[2])
+
+
+def test_nonfinite_xi_line_batched():
+    dims = [(60, 9, 8), (128, 9, 8), (140, 9, 8), (200, 9, 8), (300, 9, 8)]
+    out = []
+    for value in (0.25, np.nan):
+        b, keep = Batch(dims, "c6c"), []
+        for i, d in enumerate(dims):
+            z = fields.batch_box(d, 7 + i, device="cuda")
+            z["u"][1, 5, 7, d[0] // 3] = value
+            z["jbn"] = Operator(*d, "c6c").jacobeano(z["x"])
+            dvel, div = (torch.empty(s + d[::-1], dtype=torch.float64, device="cuda")
+                         for s in ((9,), ()))
+            b.bind(i, z["u"], z["jbn"], z["phi"], dvel, div, z["ih"], z["dxyz"], z["dt"])
+            keep.append((z, dvel, div))
+        b.stage()
+        torch.cuda.synchronize()
+        out.append([k[1][1].cpu().numpy() for k in keep])  # dv/dxi
+    for clean, got in zip(*out):
+        assert_line_only(got, clean, (5, 7))
 
 
 @pytest.mark.parametrize("value", [1e160, 1e200, -1e200, np.inf])
