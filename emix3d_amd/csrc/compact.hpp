@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "emx_internal.hpp"
+#include "dealing.hpp"
 
 namespace emx {
 
@@ -180,23 +181,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Line group of workgroup bxp (of gx along the lines) for LG lines per
-// wavefront.  A group of 8 doubles (64 bytes) shares each 128-byte cache
-// line with its neighbour.  Workgroups go to the eight XCDs round robin,
-// each XCD with its own L2, so the two halves of a line go to workgroups
-// whose ids differ by 8: the same XCD, dispatched together.
-template <int LG>
-__device__ __forceinline__ int line_group(int bxp, int gx) {
-  if constexpr (LG >= 16) {
-    return bxp;
-  } else {
-    const int base = bxp & ~15;
-    if (base + 16 > gx) return bxp;  // the last, incomplete set of 16
-    const int r = bxp & 15;
-    return base + 2 * (r & 7) + (r >> 3);
-  }
 }
 
 // Thomas factors and carry multipliers of the wavefront kind, staged in
@@ -662,50 +646,13 @@ __device__ __forceinline__ void lines_strided_body(const Prob& prob, const LineT
   }
 }
 
-// Workgroup local (of ngroup in its grid) -> line group g, row-major over
-// (group along the lines, outer index).  A grid's rows start anywhere in a
-// 128-byte cache line (its nx is any size), so neighbouring groups along a
-// row share a cache line at every point.  Workgroups go to the eight XCDs
-// round robin, each XCD with its own L2: within each set of 8K workgroups
-// (K = 16, fewer in the grid's last set), XCD x takes the K consecutive
-// groups xK .. xK+K-1, in order, so that all but one of their shared lines
-// are fetched once into that XCD's L2 and read there by the neighbour
-// dispatched next.  A bijection on [0, ngroup): the last local % 8 ids of
-// the grid keep their own group.
-__device__ __forceinline__ int xcd_run_group(int local, int ngroup) {
-  constexpr int K = 16;
-  const int base = local & ~(8 * K - 1);
-  const int k = min(K, (ngroup - base) >> 3);  // groups per XCD in this set
-  const int r = local - base;
-  if (r >= 8 * k) return local;
-  return base + (r & 7) * k + (r >> 3);
-}
-
-// run: line groups are dealt by xcd_run_group, for launches of more
-// workgroups than the chip holds at once.  Rows that start inside a cache
-// line share it with their neighbours (stage at 187 x 151 x 129: 1183 us
-// round robin, 1139 us in runs), and where they do not, a run's neighbouring
-// segments still arrive in order (256^3: 4165 and 4073 us).  A small launch
-// would only pay for the divisions (64^3 gradient and divergence: 43.2 us
-// round robin, 43.7 us in runs).
+// One workgroup per line group and outer index (deal_lines) and part.
 template <int S, int C, int LG, class Prob>
 __global__ void __launch_bounds__(1024)
 k_lines_strided(Prob prob, LineTab T, int nlanes, long long si, long long so,
                 long long sl, double ih, int run) {
   int part = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
-  if (run) {
-    int g;
-    if constexpr (interleaves<Prob>::value) {
-      g = xcd_run_group(bx + gridDim.x * (by + gridDim.y * part),
-                        gridDim.x * gridDim.y * gridDim.z);
-      part = g % gridDim.z;
-      g /= gridDim.z;
-    } else {
-      g = xcd_run_group(bx + gridDim.x * by, gridDim.x * gridDim.y);
-    }
-    bx = g % gridDim.x;
-    by = g / gridDim.x;
-  }
+  deal_lines<LG, interleaves<Prob>::value>(run, gridDim.x, gridDim.y, gridDim.z, bx, by, part);
   lines_strided_body<S, C, LG>(parts_of<Prob>::get(prob, part), T, nlanes, si, so, sl, ih, bx, by);
 }
 
@@ -942,7 +889,7 @@ __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& 
   const int tid = threadIdx.x;
   const int li = tid % LG;
   const int c = tid / LG;
-  const int i = line_group<LG>(bx, gridDim.x) * LG + li;
+  const int i = bx * LG + li;
   const bool act = i < nlanes && c < P;
   const int ic = i < nlanes ? i : nlanes - 1;
   const long long base = (long long)ic * si + (long long)by * so;
@@ -1096,7 +1043,7 @@ __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& 
   if (act && m > 0) prob.template store<C, XI>(base + (long long)s * sl, XI ? 1 : sl, m, v);
 }
 
-// Parts and run as in k_lines_strided.  Lines of up to 256 points take chunks
+// Parts and run as in k_lines_strided (deal_lines).  Lines of up to 256 points take chunks
 // of four and 16 lines per workgroup (8 lines: 119 us for the solve at 128^3
 // against 100 us, the tables being staged twice as often), up to 512 points
 // chunks of eight and 8 lines, as two tiles of 16 lines of 512 points would
@@ -1106,19 +1053,7 @@ __global__ void __launch_bounds__(C == 4 && LG == 16 ? 1024 : 512) __attribute__
 k_lines_adj(Prob prob, LineTab T, int nlanes, long long si, long long so, long long sl,
             double ih, int run) {
   int part = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
-  if (run) {
-    int g;
-    if constexpr (interleaves<Prob>::value) {
-      g = xcd_run_group(bx + gridDim.x * (by + gridDim.y * part),
-                        gridDim.x * gridDim.y * gridDim.z);
-      part = g % gridDim.z;
-      g /= gridDim.z;
-    } else {
-      g = xcd_run_group(bx + gridDim.x * by, gridDim.x * gridDim.y);
-    }
-    bx = g % gridDim.x;
-    by = g / gridDim.x;
-  }
+  deal_lines<LG, interleaves<Prob>::value>(run, gridDim.x, gridDim.y, gridDim.z, bx, by, part);
   lines_adj_body<C, LG, XI>(parts_of<Prob>::get(prob, part), T, nlanes, si, so, sl, ih, bx, by);
 }
 
