@@ -867,11 +867,17 @@ k_lines_tile(Prob prob, LineTab T, int nlanes, long long si, long long so,
 // at 128^3: 56 us a direction before, 42-46 us now (3.3 TB/s).
 constexpr int ADJ_EDGE = 4;  // rows at either end of B^T that differ
 
+// LDS tiles of the transposed solve: one where a single field needs no
+// second, or where two whole lines' tiles of 16 lanes of 512 points would
+// take all of a CU's LDS (another barrier per field instead).
+template <int C, int LG, int NV>
+constexpr int adj_tiles() { return NV == 1 || (C == 8 && LG == 16) ? 1 : 2; }
+
 template <int C, int LG, bool XI, class Prob>
 __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& T, int nlanes,
                                                long long si, long long so, long long sl,
                                                double ih, int bx, int by) {
-  constexpr int NV = Prob::NV;
+  constexpr int NV = Prob::NV, TILES = adj_tiles<C, LG, NV>();
   extern __shared__ double lds[];
   const int n = T.n, P = T.P, K = T.K, KB = T.KB;
   const int ntab = 5 * n + 1;
@@ -885,7 +891,7 @@ __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& 
   double* s_wb = s_wf + P * KB;         // [P*KB]
   double* s_be = s_wb + P * KB;         // [2*ADJ_EDGE][7]: rows 0..3 and n-4..n-1 of B^T
   double* rA = s_be + 2 * ADJ_EDGE * 7; // forward carries [NV][P][LG], then tile [n][LG]
-  double* rB = rA + region;             // backward carries, then tile
+  double* rB = rA + region;             // backward carries, then the second tile
   const int tid = threadIdx.x;
   const int li = tid % LG;
   const int c = tid / LG;
@@ -993,9 +999,11 @@ __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& 
   const bool inner = s >= ADJ_EDGE && s + C <= n - ADJ_EDGE;
 #pragma unroll
   for (int a = 0; a < NV; a++) {
-    // a tile is written again two fields later, past a barrier that follows
-    // its readers; the forward and backward carries lie a barrier back too
-    double* tile = (a & 1 ? rB : rA) + li;
+    // one of two tiles is written again two fields later, past a barrier that
+    // follows its readers; the forward and backward carries lie a barrier
+    // back too
+    double* tile = (TILES == 2 && (a & 1) ? rB : rA) + li;
+    if (TILES == 1 && a > 0) __syncthreads();
     if (act) {
 #pragma unroll
       for (int q = 0; q < C; q++)
@@ -1043,13 +1051,18 @@ __device__ __forceinline__ void lines_adj_body(const Prob& prob, const LineTab& 
   if (act && m > 0) prob.template store<C, XI>(base + (long long)s * sl, XI ? 1 : sl, m, v);
 }
 
-// Parts and run as in k_lines_strided (deal_lines).  Lines of up to 256 points take chunks
-// of four and 16 lines per workgroup (8 lines: 119 us for the solve at 128^3
-// against 100 us, the tables being staged twice as often), up to 512 points
-// chunks of eight and 8 lines, as two tiles of 16 lines of 512 points would
-// take all of a CU's LDS.
+// Parts and run as in k_lines_strided (deal_lines).  Lines of up to 256
+// points take chunks of four and 16 lines per workgroup (8 lines: 119 us for
+// the solve at 128^3 against 100 us, the tables being staged twice as often),
+// lines of up to 512 chunks of eight.  These take 16 lines along eta and
+// zeta, whole cache lines, if the fields are at most three (four need more
+// than the 128 registers of 1024 work-items) and at least 64 workgroups are
+// left: one field along eta of 128 x 512 x 33 29 us with 8 lines and 23 us
+// with 16, along zeta of 33 x 16 x 500 (48 workgroups) 11.2 and 14.8 us.
+// Along xi, where a line is contiguous, 8 lines (the divergence's adjoint at
+// 300 x 7 x 300: 64 us, 73 us with 16).
 template <int C, int LG, bool XI, class Prob>
-__global__ void __launch_bounds__(C == 4 && LG == 16 ? 1024 : 512) __attribute__((amdgpu_waves_per_eu(C == 4 ? adj_waves<Prob>::value : 2)))
+__global__ void __launch_bounds__(LG == 16 ? 1024 : 512) __attribute__((amdgpu_waves_per_eu(C == 4 ? adj_waves<Prob>::value : 2)))
 k_lines_adj(Prob prob, LineTab T, int nlanes, long long si, long long so, long long sl,
             double ih, int run) {
   int part = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
@@ -1269,23 +1282,28 @@ int launch_lines_adj_as(emx_ctx* ctx, int dir, const Prob& prob, double ih) {
   const LineTab& T = ctx->adj[dir];
   LaunchTimer timer(ctx, Prob::label(), dir, prob.bytes_pt() * (double)ctx->d.N());
   using Part = std::decay_t<decltype(parts_of<Prob>::get(prob, 0))>;
-  auto go = [&](auto kern, int LG) {
+  auto go = [&](auto kern, int LG, int tiles) {
     dim3 grid((g.nlanes + LG - 1) / LG, g.nouter, parts_of<Prob>::count(prob));
     const int threads = ((T.P * LG + 63) / 64) * 64;
     const size_t lds = (size_t)(5 * T.n + 1 + 2 * T.P * T.KB + 2 * ADJ_EDGE * 7 +
-                                2 * std::max(Part::NV * T.P, T.n) * LG) * sizeof(double);
+                                (std::max(Part::NV * T.P, T.n) +
+                                 (tiles == 2 ? std::max(Part::NV * T.P, T.n) : Part::NV * T.P)) *
+                                    LG) * sizeof(double);
     if (lds > 65536)
       (void)hipFuncSetAttribute((const void*)kern,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, grid, dim3(threads), lds, ctx->stream, prob, T, g.nlanes,
                        g.si, g.so, g.sl, ih, (int)((long long)grid.x * grid.y * grid.z > 1024));
   };
-  if constexpr (XI) {
-    if (T.C == 4) go(k_lines_adj<4, 16, true, Prob>, 16);
-    else go(k_lines_adj<8, 8, true, Prob>, 8);
+  if (T.C == 4) {
+    go(k_lines_adj<4, 16, XI, Prob>, 16, adj_tiles<4, 16, Part::NV>());
   } else {
-    if (T.C == 4) go(k_lines_adj<4, 16, false, Prob>, 16);
-    else go(k_lines_adj<8, 8, false, Prob>, 8);
+    bool wide = false;
+    if constexpr (!XI && Part::NV <= 3) {
+      wide = (long long)((g.nlanes + 15) / 16) * g.nouter * parts_of<Prob>::count(prob) >= 64;
+      if (wide) go(k_lines_adj<8, 16, XI, Prob>, 16, adj_tiles<8, 16, Part::NV>());
+    }
+    if (!wide) go(k_lines_adj<8, 8, XI, Prob>, 8, adj_tiles<8, 8, Part::NV>());
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
