@@ -47,8 +47,7 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Stages nlayer 64 x 64 weight matrices (each at src[i]) into LDS with row
-// stride MLP_LDW.
+// Stages the 64 x 64 weight matrix src into LDS with row stride MLP_LDW.
 __device__ __forceinline__ void stage_square(float* lw, const float* src) {
   for (int t = threadIdx.x; t < MLP_H * MLP_H; t += blockDim.x)
     lw[(t / MLP_H) * MLP_LDW + t % MLP_H] = src[t];
@@ -418,9 +417,16 @@ k_mlp_grad(const float* P, const float* norm, const float* feat, const float* ac
              (glds[2 * MLP_GRAD_PAD + w] + glds[3 * MLP_GRAD_PAD + w]);
 }
 
+// Workgroups of k_mlp_grad for n rows: one to a compute unit, each wavefront
+// at least one 16-row tile.  Their partial sums are the work area.
+static int mlp_grad_blocks(int n) {
+  const int tiles = (int)(((long long)n + 15) / 16);
+  return std::min(256, (tiles + MG_WAVES - 1) / MG_WAVES);
+}
+
 // grad[w] = the sum of the nblk partials: 64 values per workgroup, the
-// partials over its four wavefronts (32 values' columns are adjacent in
-// memory, so each read takes whole cache lines).
+// partials over its sixteen wavefronts (the 64 values are adjacent in memory,
+// so each read takes whole cache lines).
 __global__ void __launch_bounds__(1024)
 k_mlp_reduce(const float* part, int nblk, float* grad) {
   __shared__ float red[16][64];
@@ -472,12 +478,8 @@ int emx_mlp_forward_f32(const float* params, const float* norm, const float* fea
   return EMX_OK;
 }
 
-// Covers the partial sums (at most 256, and one per 64 rows) for every n.
-size_t emx_mlp_backward_work(int n) {
-  const int chunk = 256;
-  const size_t nblk = (size_t)((n + chunk - 1) / chunk);
-  return (size_t)n * emx::MLP_ACT + nblk * emx::MNP;
-}
+// The partial sums of every workgroup.
+size_t emx_mlp_backward_work(int n) { return (size_t)emx::mlp_grad_blocks(n) * emx::MNP; }
 
 int emx_mlp_backward_f32(const float* params, const float* norm, const float* feat,
                          const float* act, const float* dnu, int n, float* grad, float* work,
@@ -491,10 +493,7 @@ int emx_mlp_backward_f32(const float* params, const float* norm, const float* fe
                    emx_mlp_backward_work(n));
     return EMX_ERR_SIZE;
   }
-  // one workgroup of four wavefronts per compute unit, each wavefront at
-  // least one 16-row tile; the partials fit the work area for every n
-  const int tiles = (n + 15) / 16;
-  const int nblk = std::min(256, (tiles + emx::MG_WAVES - 1) / emx::MG_WAVES);
+  const int nblk = emx::mlp_grad_blocks(n);
   const size_t lds = (size_t)4 * emx::MLP_GRAD_PAD * sizeof(float);
   hipStream_t st = (hipStream_t)stream;
   EMX_TRY_HIP(hipFuncSetAttribute((const void*)emx::k_mlp_grad,
