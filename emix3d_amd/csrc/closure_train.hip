@@ -107,7 +107,8 @@ k_mlp_forward(const float* P, const float* norm, const float* feat, int n, float
       for (int s = 0; s < 3; s++) {
         const int k = 4 * s + g;
         const float f = feat[row + (k < MLP_IN ? k : 0)];
-        x[t][s] = (f - shift[s]) * scale[s];
+        // a zero row takes no part, also where feature 0 is not finite
+        x[t][s] = k < MLP_IN ? (f - shift[s]) * scale[s] : 0.0f;
       }
     }
     // keeps the pre-activations of a layer and forms the next layer's input

@@ -5,7 +5,9 @@
     line, for every chunk length of the wavefront kind, alone and batched;
   * the level set's reinitialisation where phi0^2 + dmin^2 overflows (a
     spacing that freezes its points, a level set far from any interface)
-    against the oracle, 1e-12 normwise relative.
+    against the oracle, 1e-12 normwise relative;
+  * an infinite feature of the closure's training pass gives infinities of
+    the weights' signs in its row's first layer, and leaves the other rows.
 """
 import numpy as np
 import pytest
@@ -13,6 +15,8 @@ import torch
 
 from conftest import normwise_rel
 from emix3d_amd import Batch, Operator, fields
+from emix3d_amd.api import mlp_forward_f32
+from test_oracle_mlp import rand_norm, rand_params
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +118,17 @@ def test_reinit_far_from_any_interface(oracle, value):
     ref = oracle.ls_reinit(phi, jbn, dmins, dxyz, float(dmins.min()))
     assert normwise_rel(ref / value, np.ones_like(phi)) <= 7e-15
     assert normwise_rel(p.cpu().numpy() / value, np.ones_like(phi)) <= 7e-15
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf])
+@pytest.mark.parametrize("feature", [0, 1, 9])
+def test_infinite_feature(feature, value):
+    P, norm = rand_params(31), rand_norm(32)
+    feat = np.random.default_rng(feature).standard_normal((50, 10)).astype(np.float32)
+    clean, _ = mlp_forward_f32(dev(P), dev(norm), dev(feat))
+    feat[33, feature] = value
+    act, _ = mlp_forward_f32(dev(P), dev(norm), dev(feat))
+    act, clean = act.cpu().numpy(), clean.cpu().numpy()
+    w = P[:640].reshape(64, 10)[:, feature] * norm[10 + feature]
+    assert np.array_equal(act[33, :64], np.copysign(np.float32(np.inf), w * value))
+    assert np.array_equal(np.delete(act, 33, 0), np.delete(clean, 33, 0))
