@@ -31,7 +31,7 @@ struct BatchShape {
 // lg lines per wavefront of the strided kind, or lg = 0 for the wavefront
 // kind (one wavefront per line, direction 0 only: its lines are contiguous,
 // so each load instruction of a wave reads consecutive points), where each
-// box takes the shortest of the chunk lengths 1, 2, 4, 8 up to C that fits.
+// box takes the shortest of the chunk lengths 1, 2, 3, 4, 8 up to C that fits.
 static const BatchShape kBatchShapes[] = {{8, 4},  {8, 8},   {16, 4}, {16, 8},
                                           {32, 4}, {32, 8},  {64, 8}, {64, 16},
                                           {0, 1},  {0, 2},   {0, 4},  {0, 8}};
@@ -493,8 +493,13 @@ int emx_batch_tune(emx_batch* b, int reps) {
   for (int d = 0; d < 3 && rc == EMX_OK; d++) {
     float best = 1e30f;
     emx::BatchShape pick = b->shape[d];
+    bool wave_timed = false;
     for (const auto& s : emx::kBatchShapes) {
       if (!emx::shape_fits(b, d, s)) continue;
+      // the wavefront kind's kernel and chunks follow the boxes' lines: every
+      // shape of it that fits is the same launch
+      if (s.lg == 0 && wave_timed) continue;
+      wave_timed |= s.lg == 0;
       rc = emx::quiesce(b);  // the previous shape's launches read the tables
       if (rc == EMX_OK) rc = emx::plan_lines(b, d, s);
       if (rc != EMX_OK) break;

@@ -223,7 +223,7 @@ int emx_batch_bind(emx_batch* b, int i, const double* u, const double* jbn, doub
 /* Line-solver shape of direction dir: lg lines per wavefront (8, 16, 32,
  * 64) and C points per work-item; built pairs (8,4) (8,8) (16,4) (16,8)
  * (32,4) (32,8) (64,8) (64,16).  lg = 0 (direction 0 only) is one wavefront per line,
- * each box with the shortest of 1, 2, 4, 8 points per lane up to C that
+ * each box with the shortest of 1, 2, 3, 4, 8 points per lane up to C that
  * fits its lines (C = 1, 2, 4, 8; every line at most 64*C points): the
  * default for direction 0. */
 int emx_batch_set_plan(emx_batch* b, int dir, int lg, int C);
