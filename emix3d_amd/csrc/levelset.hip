@@ -305,24 +305,6 @@ __device__ __forceinline__ double weno5(double b1, double b2, double b3, double 
   return weno5_e(b3, b2 - b1, b3 - b2, b4 - b3, b5 - b4);
 }
 
-// Backward difference of phi along axis `ax` at point (x,y,z), with the
-// index-0 rule of Dev1thO_Downwind (lsTools.cu:53-95).
-__device__ __forceinline__ double bdiff(const double* phi, PDims g, int ax,
-                                        int x, int y, int z, double ih) {
-  const long long sxy = (long long)g.x * g.y;
-  const long long id = (long long)x + (long long)g.x * y + sxy * z;
-  if (ax == 0) {
-    if (x == 0) return ih * (gref(phi + id + 1) - gref(phi + id));
-    return ih * (gref(phi + id) - gref(phi + id - 1));
-  }
-  if (ax == 1) {
-    if (y == 0) return ih * (gref(phi + id + g.x) - gref(phi + id));
-    return ih * (gref(phi + id) - gref(phi + id - g.x));
-  }
-  if (z == 0) return ih * (gref(phi + id + sxy) - gref(phi + id));
-  return ih * (gref(phi + id) - gref(phi + id - sxy));
-}
-
 // ---------------------------------------------------------------------------
 // Level-set reinitialisation (cuReinitLsJB, lsTransportEc.cu:422-676).
 
@@ -537,9 +519,13 @@ k_ls_reinit_stage(const double* src, const double* P, const double* dmin, const 
     double z5 = bz[4];
     if (STAGE < 2 && (z < 3 || z > g.z - 4)) {
       edge_bd(bz, z, g.z);
-      // on the last plane L's fifth operand is the z difference one row down
-      // (id_kp2 = id_jm1, lsTools.cu:636)
-      z5 = z == g.z - 1 ? bdiff(src, g, 2, xc, yc == 0 ? yc : yc - 1, z, sZ) : bz[4];
+      z5 = bz[4];
+      if (z == g.z - 1) {
+        // on the last plane L's fifth operand is the z difference one row
+        // down (id_kp2 = id_jm1, lsTools.cu:636)
+        const unsigned row = (unsigned)xc + sy * (unsigned)(yc == 0 ? 0 : yc - 1);
+        z5 = sZ * (ld(src, (row + (unsigned)z * sz) * 8u) - ld(src, (row + (unsigned)(z - 1) * sz) * 8u));
+      }
     }
     const double rx = godunov_axis(bx, bx[4]), ry = godunov_axis(by, by[4]),
                  rz = godunov_axis(bz, z5);
