@@ -5,8 +5,9 @@
 // Kernel shapes (CDNA4, 64-wide wavefronts):
 //  * k_lines_wave    -- one wavefront per line; lane c owns C consecutive
 //    points.  Used for xi lines, which are contiguous in memory: a wave
-//    reads one line with unit-stride loads.  Chunk carries travel through
-//    six shuffle steps of a weighted prefix scan.
+//    reads one line with unit-stride loads.  Chunk carries travel through a
+//    weighted prefix scan over the lanes, of up to six steps (lane shifts
+//    for distances 1 and 2, shuffles beyond).
 //  * k_lines_strided -- 64 neighbouring lines (consecutive i) per
 //    workgroup, the line split over up to 16 waves, C points per lane.
 //    Used for eta/zeta lines: every load instruction of a wave reads 64

@@ -276,8 +276,7 @@ int emx_adam_f32(float* params, const float* grad, float* m, float* v, int n, fl
  * exact transpose of the forward entry it names (same scheme and metric
  * projection), for gradient-based use and the learned closure's training.
  * Lines of at most 512 points in every direction (EMX_ERR_SIZE otherwise).
- * Outputs are overwritten; they may hold intermediate results meanwhile, so
- * no output may overlap an input or another output. */
+ * Outputs are overwritten. */
 
 /* out = D^T g for D = emx_deriv along dir with inverse spacing inv_h. */
 int emx_deriv_adj(emx_ctx* ctx, int dir, const double* g, double* out,
@@ -298,7 +297,8 @@ int emx_divergence_adj(emx_ctx* ctx, const double* rs_bar, const double* rsv_bar
 /* Transpose of the linearisation of emx_flux_div_all about (um, u, vis,
  * dvel) (pres enters linearly; jbn is fixed): from the adjoints of rs (5
  * fields) and rsv (5 fields; 1 and 5 unused) to those of um (5, the first
- * is zero), u (3), pres, vis and dvel (9). */
+ * is zero), u (3), pres, vis and dvel (9).  The outputs hold intermediate
+ * results meanwhile: none may overlap an input or another output. */
 int emx_flux_div_all_adj(emx_ctx* ctx, const double* rs_bar, const double* rsv_bar,
                          const double* um, const double* u, const double* vis,
                          const double* jbn, const double* dvel, double ihx,
