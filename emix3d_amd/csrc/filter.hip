@@ -16,7 +16,6 @@ namespace emx {
 struct ProbFilter {
   static constexpr int NV = 1;
   static const char* label() { return "filter"; }
-  double bytes_pt() const { return 8.0 * 4; }  // f, J, 1/J in; f out
   double* f;
   const double* jac;
   const double* ijac;
