@@ -106,9 +106,9 @@ k_mlp_forward(const float* P, const float* norm, const float* feat, int n, float
 #pragma unroll
       for (int s = 0; s < 3; s++) {
         const int k = 4 * s + g;
-        const float f = feat[row + (k < MLP_IN ? k : 0)];
-        // a zero row takes no part, also where feature 0 is not finite
-        x[t][s] = k < MLP_IN ? (f - shift[s]) * scale[s] : 0.0f;
+        float f = 0.0f;  // of the zero rows: no feature, which may not be finite
+        if (k < MLP_IN) f = feat[row + k];
+        x[t][s] = (f - shift[s]) * scale[s];
       }
     }
     // keeps the pre-activations of a layer and forms the next layer's input
