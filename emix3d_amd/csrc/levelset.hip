@@ -250,18 +250,23 @@ __device__ __forceinline__ double recip_nr(double x) {
 }
 
 // 1/sqrt(x) for x > 0, by the same third-order step: r (1 + e/2 + 3 e^2/8),
-// e = 1 - x r^2.  At infinity r = 0, and the product that forms e takes the
-// largest number instead (0, not NaN): the result is 0.
+// e = 1 - x r^2, given xr = x r.
+__device__ __forceinline__ double rsqrt_step(double r, double xr) {
+  const double e = __builtin_fma(-xr, r, 1.0);
+  return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+}
+
+// At infinity r = 0, and the largest number takes the place of x in x r (0,
+// not NaN): the result is 0.
 __device__ __forceinline__ double rsqrt_nr(double x) {
   const double r = __builtin_amdgcn_rsq(x);
-  const double e = __builtin_fma(-(__builtin_fmin(x, 0x1.fffffffffffffp1023) * r), r, 1.0);
-  return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+  return rsqrt_step(r, __builtin_fmin(x, 0x1.fffffffffffffp1023) * r);
 }
 
 // sqrt(x) for x >= 0: x/sqrt(x) and one residual step where x is a positive
 // finite number; 0, infinity and NaN are their own roots.
 __device__ __forceinline__ double sqrt_nr(double x) {
-  const double r = rsqrt_nr(x);
+  const double r0 = __builtin_amdgcn_rsq(x), r = rsqrt_step(r0, x * r0);
   const double s = x * r;
   const double t = __builtin_fma(__builtin_fma(-s, s, x), 0.5 * r, s);
   return __builtin_amdgcn_class(x, 0x180) ? t : x;
